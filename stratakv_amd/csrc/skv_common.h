@@ -71,6 +71,20 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
 }
 
+// Two fp32 values as three bf16 parts each, packed two to a word, whose sum is
+// the value exactly (normal values: 24 significant bits = 8 + 8 + 8): part 0 is
+// the top 16 bits, part 1 the top 16 bits of the exact remainder, part 2 the
+// rest.  A part of an infinity or NaN is the value itself, the others NaN.
+__device__ __forceinline__ void split3_pair(float v0, float v1, uint32_t (&w)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const uint32_t b0 = __float_as_uint(v0), b1 = __float_as_uint(v1);
+        w[i] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);   // high halves: b1 << 16 | b0 >> 16
+        v0 -= __uint_as_float(b0 & 0xffff0000u);
+        v1 -= __uint_as_float(b1 & 0xffff0000u);
+    }
+}
+
 // Unpack 8 bf16 held in a 16-byte vector into fp32.
 __device__ __forceinline__ void unpack8(const uint4& w, float (&f)[8]) {
     f[0] = bf16_lo(w.x); f[1] = bf16_hi(w.x);
@@ -134,17 +148,19 @@ __device__ __forceinline__ float swap8_sum(float a, float b) {
 }
 
 // Reduce-scatter of N per-lane values over the lanes that share lane bits
-// 0 .. LO-1 (the groups l, l + 2^LO, ...; LO = 3 or 4): every exchange keeps
+// 0 .. LO-1 (the groups l, l + 2^LO, ...; LO = 3, 4 or 5): every exchange keeps
 // complementary halves, so afterwards lane l holds, in v[0 .. N/2^(6-LO)), the
 // group sums of values (l >> LO) * N/2^(6-LO) + i.  Each sum is the same
 // pairwise tree for every value: bit 5 pairs first, then bit 4, then bit 3.
 template <int N, int LO>
 __device__ __forceinline__ void reduce_scatter_high_bits(float (&v)[N]) {
-    static_assert((LO == 3 || LO == 4) && N % (1 << (6 - LO)) == 0, "reduce-scatter shape");
+    static_assert(LO >= 3 && LO <= 5 && N % (1 << (6 - LO)) == 0, "reduce-scatter shape");
 #pragma unroll
     for (int i = 0; i < N / 2; ++i) v[i] = swap32_sum(v[i], v[i + N / 2]);
+    if constexpr (LO <= 4) {
 #pragma unroll
-    for (int i = 0; i < N / 4; ++i) v[i] = swap16_sum(v[i], v[i + N / 4]);
+        for (int i = 0; i < N / 4; ++i) v[i] = swap16_sum(v[i], v[i + N / 4]);
+    }
     if constexpr (LO == 3) {
 #pragma unroll
         for (int i = 0; i < N / 8; ++i) v[i] = swap8_sum(v[i], v[i + N / 8]);

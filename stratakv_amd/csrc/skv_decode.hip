@@ -44,6 +44,7 @@
 #include <cstdio>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <unordered_map>
 
 namespace skv {
@@ -82,6 +83,12 @@ struct DecodeParams {
     int merge_cw;          // output columns per merge workgroup (a multiple of 64)
     int max_slots;         // (range, head group) pairs the workspace holds partials for
     int seg_cost;          // stream-K: blocks' worth of time charged per segment start (see WorkSplit)
+    // The split counts units of 16 tokens on the MFMA path (whatever the pool's
+    // block size) and blocks on the generic one, at most max_units of a
+    // sequence; max_tokens positions of it lie in its table (ANY instances).
+    int max_units, max_tokens;
+    int bs_log2;           // ANY instances: log2(block size)
+    int q_fp32;            // ANY instances: fp32 queries
 };
 
 constexpr int kMaxHeadDim = 512;
@@ -95,10 +102,13 @@ __device__ __forceinline__ int seq_len(const DecodeParams& p, int b) {
     return p.lens != nullptr ? p.lens[b] : p.single_len;
 }
 
-__device__ __forceinline__ int seq_blocks(const DecodeParams& p, int b) {
+// Units of sequence b.  UNIT: tokens per unit when it is a constant (a shift
+// instead of an integer division before the split), 0 = the block size.
+template <int UNIT>
+__device__ __forceinline__ int seq_units(const DecodeParams& p, int b) {
     const int L = seq_len(p, b);
     if (L <= 0) return 0;
-    return std::min(cdiv(L, p.bs), p.max_blocks);
+    return std::min((L - 1) / (UNIT > 0 ? UNIT : p.bs) + 1, p.max_units);
 }
 
 // ---------------------------------------------------------------------------
@@ -144,13 +154,14 @@ struct WorkSplit {
     }
 };
 
+template <int UNIT>
 __device__ WorkSplit build_split(const DecodeParams& p, int* P_s, bool stream_k) {
     const int lane = threadIdx.x;
     if (lane < 64) {  // wavefront 0 of the workgroup scans
         int carry = 0;
         for (int b0 = 0; b0 < p.B; b0 += 64) {
             const int b = b0 + lane;
-            int v = b < p.B ? seq_blocks(p, b) : 0;
+            int v = b < p.B ? seq_units<UNIT>(p, b) : 0;
             if (blockIdx.x == 0 && p.out != nullptr) {
                 // Sequences without context produce zeros (workgroup 0 writes them).
                 uint64_t empty = __ballot(b < p.B && v == 0);
@@ -241,7 +252,9 @@ __device__ __forceinline__ void store_scaled(float* o, const float* x, float sc)
 }
 
 // ---------------------------------------------------------------------------
-// MFMA path: block_size 16, head_dim 64 or 128, G in {1, 2, 4, 8, 16}.
+// MFMA path: block_size 16, head_dim 64 or 128, G in {1, 2, 4, 8, 16}; the ANY
+// instances take every other block size that is a power of two, head_dim up to
+// 256 in multiples of 8 and G up to 16, padded to HD and G (below).
 // Coalesced (V) layout: lane (r, c) = (lane / CH, lane % CH) holds rows
 //   i*RPI + r (i < TPL) of a block, elements [8c, 8c + 8).
 // MFMA layout: lane (t, j) = (lane % 16, lane / 16); the K operand of MFMA cc
@@ -256,21 +269,41 @@ __device__ __forceinline__ void store_scaled(float* o, const float* x, float sc)
 // Wavefronts per SIMD the MFMA kernel is launched with (see launch_mfma_shape);
 // also its register budget (launch bound).
 constexpr int mfma_waves_per_simd(int HD, int G) { return HD == 64 && G < 16 ? 2 : 1; }
+// Chunk position of row `row` in the K tile (see above).
+template <int CH>
+__device__ __forceinline__ int k_swizzle(int row) { return CH >= 16 ? row : ((row >> 1) & 7); }
 
 // SPLIT: short tables (at most WPW * NBUF blocks per sequence).  Workgroup
 // = one (sequence, kv head) segment; its WPW wavefronts take consecutive
 // sub-ranges of at most NBUF blocks, so every K/V load of the segment is in
 // flight at once, and merge their partials through LDS (no merge launch).
-template <int HD, int G, bool QF32, int WPW, int NBUF, bool SPLIT = false>
+//
+// ANY: the pool's own head_dim p.HD <= HD (lanes of the chunks past it load
+// chunk 0 again and count as zeros), p.NH <= G query heads per kv head (the
+// padded ones have zero queries and store nothing) and a block size of
+// 2^p.bs_log2 tokens.  ANY = 1: blocks of 16 tokens and more, a unit of 16 is
+// part of one table entry and read through one descriptor as above.  ANY = 2:
+// smaller blocks, a unit spans several entries, so every lane addresses its
+// rows itself: a lane's window entry holds the byte offset of its block, read
+// per row with a lane shuffle, and issue()'s result has one bit per table
+// entry of the unit.  fp32 queries are split exactly into three bf16 parts (8 + 8 + 8
+// significant bits, three MFMAs), the precision of the generic kernel these
+// instances take over from: its lanes read one K row each with 2-byte loads
+// and its K/V rows once per query head, 1,878 us for 24 sequences of 200-4,096
+// tokens, 24 query / 8 kv heads of 128 (181 MB, 0.10 TB/s); 37.6 us here
+// (4.8 TB/s, HBM-bound as the tuned shapes).
+template <int HD, int G, bool QF32, int WPW, int NBUF, bool SPLIT = false, int ANY = 0>
 __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_mfma_kernel(DecodeParams p) {
     constexpr int BS = 16;
     constexpr int CH = HD / 8;      // 16-byte chunks per row
     constexpr int RPI = 64 / CH;    // rows per coalesced load instruction
     constexpr int TPL = BS / RPI;   // rows per lane per block (coalesced layout)
     constexpr int NMF = HD / 32;    // MFMAs per block for q.k
-    constexpr int QP = QF32 ? 2 : 1;
+    constexpr int QP = ANY ? 3 : QF32 ? 2 : 1;
     static_assert(CH * RPI == 64 && RPI * TPL == BS && NMF * 4 == CH, "lane layout");
     static_assert(G >= 1 && G <= 16, "group size");
+    const int hd = ANY ? p.HD : HD;   // head_dim and query heads per kv head of the call
+    const int gq = ANY ? p.NH : G;
 
     // Per-wavefront LDS: the WPW wavefronts of a workgroup serve the same
     // range for WPW consecutive kv heads and only meet at the work split.
@@ -288,7 +321,8 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
     float (*h_s)[16] = h_all[wv];
     const int r = lane / CH, c = lane % CH;
     const int t = lane & 15, j = lane >> 4;
-    auto swz = [](int row) { return CH == 16 ? row : ((row >> 1) & 7); };
+    auto swz = [](int row) { return k_swizzle<CH>(row); };
+    const bool in_hd = !ANY || c * 8 < hd;   // this lane's chunk exists
     const int Hkv = p.Hkv;
     const int w = blockIdx.x * WPW + wv;    // Hkv % WPW == 0: one range per workgroup
     const int kvh = SPLIT ? static_cast<int>(blockIdx.x % Hkv) : w % Hkv;
@@ -315,9 +349,9 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
         for (int cc = 0; cc < NMF; ++cc) {
             qa[cc][0] = qa[cc][1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             qh[cc] = u32x4_t{0u, 0u, 0u, 0u};
-            if (t < G) {
-                const int64_t qoff = (static_cast<int64_t>(bq) * p.Hq + kvh * G + t) * HD + (4 * cc + j) * 8;
-                if constexpr (QF32) {
+            if (t < gq && (!ANY || (4 * cc + j) * 8 < hd)) {
+                const int64_t qoff = (static_cast<int64_t>(bq) * p.Hq + kvh * gq + t) * hd + (4 * cc + j) * 8;
+                if (ANY ? p.q_fp32 != 0 : QF32) {
                     const float4* qp = reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + qoff);
                     qa[cc][0] = qp[0];
                     qa[cc][1] = qp[1];
@@ -329,9 +363,9 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
     };
     if constexpr (SPLIT) load_q_raw(static_cast<int>(blockIdx.x / Hkv));
 
-    const WorkSplit split = build_split(p, P_s, !SPLIT);
+    const WorkSplit split = build_split<BS>(p, P_s, !SPLIT);
     if (!SPLIT && range >= split.used) return;
-    const int64_t row_stride = static_cast<int64_t>(Hkv) * HD;
+    const int64_t row_stride = static_cast<int64_t>(Hkv) * hd;
     const int block_bytes = static_cast<int>(BS * row_stride * 2);
     int range_lo = SPLIT ? 0 : split.lo(range);
     int range_hi = SPLIT ? 0 : split.lo(range + 1);
@@ -345,7 +379,14 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
     int pos = range_lo;
     const int end = SPLIT ? range_hi : std::min(range_hi, split.total);
     if (!SPLIT) b = find_seq(P_s, p.B, pos);
-    const int h0 = kvh * G;
+    const int h0 = kvh * gq;
+    // ANY = 2: a unit covers 2^per_unit table entries; ANY = 1: 2^per_entry
+    // units share one.
+    const int per_unit = ANY == 2 ? 4 - p.bs_log2 : 0;
+    const int per_entry = ANY == 1 ? p.bs_log2 - 4 : 0;
+    auto unit_entry = [&](int kb) -> int {   // first table entry of unit kb
+        return ANY == 2 ? kb << per_unit : ANY == 1 ? kb >> per_entry : kb;
+    };
 
     while (!SPLIT || pos < end) {
         const int seg_lo = SPLIT ? P_s[b] : seg_first(P_s, b, p.seg_cost), seg_hi = P_s[b + 1];
@@ -358,7 +399,7 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
         const int stop = std::min(end, seg_hi);
         const int kb1 = stop - seg_lo;
         const int L = seq_len(p, b);
-        const int Leff = std::min(L, nb * BS);
+        const int Leff = ANY ? std::min(L, p.max_tokens) : std::min(L, nb * BS);
         const int32_t* table = p.tables + static_cast<int64_t>(b) * p.max_blocks;
 
         // Fused append: the wavefront whose range holds the segment's last block
@@ -370,16 +411,18 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
         int kb_new = -1, i_new = 0, r_new = 0;
         int64_t new_dst = 0;
         u32x4_t knew = {0u, 0u, 0u, 0u}, vnew = {0u, 0u, 0u, 0u};
-        if (p.k_new != nullptr && kb1 == nb && L >= 1 && L <= nb * BS) {
-            const int64_t e = SPLIT ? __shfl(trow, nb - 1, 64) : table[nb - 1];
+        if (p.k_new != nullptr && kb1 == nb && L >= 1 && L <= (ANY ? p.max_tokens : nb * BS)) {
+            const int e_new = ANY ? (L - 1) >> p.bs_log2 : nb - 1;
+            const int64_t e = SPLIT ? __shfl(trow, e_new, 64) : table[e_new];
             if (e >= 0 && e < p.total_blocks) {
                 const int slot = (L - 1) - (nb - 1) * BS;
                 kb_new = nb - 1;
                 i_new = slot / RPI;
                 r_new = slot % RPI;
-                new_dst = (e * BS + slot) * row_stride + static_cast<int64_t>(kvh) * HD + c * 8;
-                if (r == r_new) {
-                    const int64_t src = (static_cast<int64_t>(b) * Hkv + kvh) * HD + c * 8;
+                const int64_t row_new = ANY ? (e << p.bs_log2) + ((L - 1) & ((1 << p.bs_log2) - 1)) : e * BS + slot;
+                new_dst = row_new * row_stride + static_cast<int64_t>(kvh) * hd + c * 8;
+                if (r == r_new && in_hd) {
+                    const int64_t src = (static_cast<int64_t>(b) * Hkv + kvh) * hd + c * 8;
                     if (p.kv_new_fp32) {
                         const float4* ks = reinterpret_cast<const float4*>(static_cast<const float*>(p.k_new) + src);
                         const float4* vs = reinterpret_cast<const float4*>(static_cast<const float*>(p.v_new) + src);
@@ -402,7 +445,25 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
 #pragma unroll
         for (int cc = 0; cc < NMF; ++cc) {
             u32x4_t hi = qh[cc], lo = {0u, 0u, 0u, 0u};
-            if constexpr (QF32) {
+            if constexpr (ANY) {
+                // x = part 0 + part 1 + part 2 exactly: each part takes the top
+                // 8 significant bits of what is left (truncation).
+                u32x4_t mid = {0u, 0u, 0u, 0u};
+                if (p.q_fp32) {
+                    const float4 a0 = qa[cc][0], a1 = qa[cc][1];
+                    const float x[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        uint32_t w[3];
+                        split3_pair(x[2 * e], x[2 * e + 1], w);
+                        hi[e] = w[0];
+                        mid[e] = w[1];
+                        lo[e] = w[2];
+                    }
+                }
+                qop[QP - 2][cc] = __builtin_bit_cast(bf16x8_t, mid);
+                qop[QP - 1][cc] = __builtin_bit_cast(bf16x8_t, lo);
+            } else if constexpr (QF32) {
                 const float4 a0 = qa[cc][0], a1 = qa[cc][1];
                 const float x[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
                 uint32_t hb[8], lb[8];
@@ -415,7 +476,7 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
                 lo = u32x4_t{lb[0] | lb[1] << 16, lb[2] | lb[3] << 16, lb[4] | lb[5] << 16, lb[6] | lb[7] << 16};
             }
             qop[0][cc] = __builtin_bit_cast(bf16x8_t, hi);
-            if constexpr (QF32) qop[QP - 1][cc] = __builtin_bit_cast(bf16x8_t, lo);
+            if constexpr (QF32 && !ANY) qop[QP - 1][cc] = __builtin_bit_cast(bf16x8_t, lo);
         }
 
         float m = -INFINITY;   // reference max of head t (log2 units), equal across j
@@ -426,36 +487,73 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[g][e] = 0.0f;
 
-        const int lane_off_b = static_cast<int>((r * row_stride + static_cast<int64_t>(kvh) * HD + c * 8) * 2);
+        const int lane_off_b = static_cast<int>((r * row_stride + static_cast<int64_t>(kvh) * hd + (in_hd ? c * 8 : 0)) * 2);
 
         // Table entries of the segment, 64 at a time: lane i holds entry tb + i
         // (tv) and tb + 64 + i (tvn, loaded one chunk ahead), so the block
         // addresses never wait on a dependent table load.
+        const int last_entry = ANY ? std::min(unit_entry(kb1 - 1) + (1 << per_unit), p.max_blocks) - 1 : kb1 - 1;
         auto table_entry = [&](int k) -> int {
-            const int kc = k < kb1 ? k : kb1 - 1;
-            if constexpr (SPLIT) return __shfl(trow, kc, 64);  // kc < nb <= max_blocks
+            const int kc = std::min(k, last_entry);
+            if constexpr (SPLIT) return __shfl(trow, kc, 64);  // kc < max_blocks <= 64
             return table[kc];
         };
-        int tb = k0;
+        int tb = unit_entry(k0);
         int tv = table_entry(tb + lane);
         int tvn = table_entry(tb + 64 + lane);
+        // ANY = 2: this lane's window entry as the byte offset of its block (0 for
+        // an entry outside the pool) and which of the window's entries exist.
+        uint64_t blk_off = 0, wmask = 0;
+        auto set_window = [&]() {
+            if constexpr (ANY == 2) {
+                const bool ok = tv >= 0 && tv < p.total_blocks;
+                blk_off = ok ? (static_cast<uint64_t>(tv) << p.bs_log2) * static_cast<uint64_t>(row_stride) * 2 : 0ull;
+                wmask = __ballot(ok);
+            }
+        };
+        set_window();
 
         // Loads of block kb into one register buffer.  Every call issues the
         // same loads, so the compiler's wait counts stay exact: a position
         // past the segment, or a table entry outside the pool, reads through
         // a buffer descriptor of size 0, whose loads return zeros without
         // touching memory.  The return value says whether the block is real.
-        auto issue = [&](int kb, u32x4_t (&kk)[TPL], u32x4_t (&vv)[TPL]) -> bool {
+        // (bool where one bit does: as a word, hd 64 / G 8 takes 240 VGPRs for 173)
+        using Ok = std::conditional_t<ANY == 2, uint32_t, bool>;
+        auto issue = [&](int kb, u32x4_t (&kk)[TPL], u32x4_t (&vv)[TPL]) -> Ok {
             const bool in_seg = kb < kb1;
             kb = in_seg ? kb : kb1 - 1;
-            if (kb - tb >= 64) {  // blocks are issued in order: advance one chunk
+            if (unit_entry(kb) - tb >= 64) {  // blocks are issued in order: advance one chunk
                 tb += 64;
                 tv = tvn;
                 tvn = table_entry(tb + 64 + lane);
+                set_window();
             }
-            const int64_t e = __builtin_amdgcn_readlane(tv, kb - tb);
+            if constexpr (ANY == 2) {
+                // Rows i * RPI + r of the unit; a row whose entry does not
+                // exist, and a unit past the segment, load row 0 of the pool
+                // (consume() does not use what they bring).
+                const int e0 = unit_entry(kb) - tb;
+#pragma unroll
+                for (int i = 0; i < TPL; ++i) {
+                    const int row = i * RPI + r;
+                    const int at = e0 + (row >> p.bs_log2);
+                    const int slot = row & ((1 << p.bs_log2) - 1);
+                    const uint64_t off = static_cast<uint32_t>(__shfl(static_cast<int>(blk_off), at, 64)) |
+                                         static_cast<uint64_t>(static_cast<uint32_t>(
+                                             __shfl(static_cast<int>(blk_off >> 32), at, 64))) << 32;
+                    const bool ok = in_seg && ((wmask >> at) & 1u) != 0;
+                    const uint64_t at_b = (ok ? off + static_cast<uint64_t>(slot) * static_cast<uint64_t>(row_stride) * 2 : 0ull) +
+                                          static_cast<uint64_t>((static_cast<int64_t>(kvh) * hd + (in_hd ? c * 8 : 0)) * 2);
+                    kk[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(p.k) + at_b));
+                    vv[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(reinterpret_cast<const char*>(p.v) + at_b));
+                }
+                return in_seg ? static_cast<uint32_t>(wmask >> e0) & ((1u << (1 << per_unit)) - 1u) : 0u;
+            }
+            const int64_t e = __builtin_amdgcn_readlane(tv, unit_entry(kb) - tb);
             const bool valid = in_seg && e >= 0 && e < p.total_blocks;
-            const int64_t base = (valid ? e : 0) * BS * row_stride;
+            const int64_t row0 = ANY == 1 ? (e << p.bs_log2) + (kb & ((1 << per_entry) - 1)) * BS : e * BS;
+            const int64_t base = (valid ? row0 : 0) * row_stride;
             const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<uint16_t*>(p.k + base), 0, valid ? block_bytes : 0, kRsrcWord3);
             const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
@@ -469,7 +567,13 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
             return valid;
         };
 
-        auto consume = [&](int kb, u32x4_t (&kk)[TPL], u32x4_t (&vv)[TPL]) {
+        // `ok`: issue()'s result for this block (not 0).
+        auto consume = [&](int kb, Ok ok, u32x4_t (&kk)[TPL], u32x4_t (&vv)[TPL]) {
+            // Whether row `row` of the unit has a block (ANY with several
+            // entries per unit; else every row of a consumed block has).
+            auto present = [&](int row) {
+                return ANY != 2 || ((static_cast<uint32_t>(ok) >> (row >> p.bs_log2)) & 1u) != 0;
+            };
             if (kb == kb_new) {  // the block that receives the appended token
 #pragma unroll
                 for (int i = 0; i < TPL; ++i) {
@@ -483,7 +587,7 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
 #pragma unroll
             for (int i = 0; i < TPL; ++i) {
                 const int row = i * RPI + r;
-                k_s[row * CH + (c ^ swz(row))] = kk[i];
+                k_s[row * CH + (c ^ swz(row))] = in_hd ? kk[i] : u32x4_t{0u, 0u, 0u, 0u};
             }
             wave_lds_sync();
             // ---- scores S[token 4j+i][head t] on the matrix cores
@@ -492,13 +596,15 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
             for (int cc = 0; cc < NMF; ++cc) {
                 const bf16x8_t a = __builtin_bit_cast(bf16x8_t, k_s[t * CH + ((4 * cc + j) ^ swz(t))]);
 #pragma unroll
-                for (int qp = 0; qp < QP; ++qp)
+                for (int qp = 0; qp < QP; ++qp) {
+                    if (ANY && qp > 0 && !p.q_fp32) continue;
                     sacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qop[qp][cc], sacc, 0, 0, 0);
+                }
             }
             const int tok = kb * BS + 4 * j;
             float s[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s[i] = tok + i < Leff ? sacc[i] * p.qscale : -INFINITY;
+            for (int i = 0; i < 4; ++i) s[i] = tok + i < Leff && present(4 * j + i) ? sacc[i] * p.qscale : -INFINITY;
             float mb = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
             // (ds_bpermute: on the LDS pipe beside the VALU work of the block,
             // measurably faster here than the VALU permlane swaps)
@@ -537,7 +643,7 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
             for (int i = 0; i < TPL; ++i) {
                 const int row = i * RPI + r;
                 u32x4_t vw = vv[i];
-                if (tail && kb * BS + row >= Leff) vw = u32x4_t{0u, 0u, 0u, 0u};
+                if ((tail && kb * BS + row >= Leff) || !present(row)) vw = u32x4_t{0u, 0u, 0u, 0u};
                 float vf[8];
                 vf[0] = bf16_lo(vw.x); vf[1] = bf16_hi(vw.x);
                 vf[2] = bf16_lo(vw.y); vf[3] = bf16_hi(vw.y);
@@ -558,18 +664,18 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
         // holds block kb + u: while one block is consumed the next NBUF - 1
         // are in flight, and no register copy forces an early wait.
         u32x4_t kbuf[NBUF][TPL], vbuf[NBUF][TPL];
-        bool okb[NBUF];
+        Ok okb[NBUF];
 #pragma unroll
         for (int u = 0; u < NBUF; ++u) okb[u] = issue(k0 + u, kbuf[u], vbuf[u]);
         for (int kb = k0; kb < kb1; kb += NBUF) {
 #pragma unroll
             for (int u = 0; u < NBUF; ++u) {
-                if (okb[u]) consume(kb + u, kbuf[u], vbuf[u]);
+                if (okb[u]) consume(kb + u, okb[u], kbuf[u], vbuf[u]);
                 okb[u] = issue(kb + u + NBUF, kbuf[u], vbuf[u]);
             }
         }
 
-        if (kb_new >= 0 && r == r_new) {  // fused append: store the new row
+        if (kb_new >= 0 && r == r_new && in_hd) {  // fused append: store the new row
             *reinterpret_cast<u32x4_t*>(p.k_pool_w + new_dst) = knew;
             *reinterpret_cast<u32x4_t*>(p.v_pool_w + new_dst) = vnew;
         }
@@ -578,7 +684,7 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
         // after which lane (r, c) holds NF consecutive (head, element) values
         // v = NF * r + i (head v / 8, dims 8c + v % 8), exactly what it stores.
         constexpr int NV = G * 8;
-        constexpr int LO = CH == 8 ? 3 : 4;
+        constexpr int LO = CH == 8 ? 3 : CH == 16 ? 4 : 5;
         constexpr int NF = NV >> (6 - LO);
         float v[NV];
 #pragma unroll
@@ -603,10 +709,11 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
 #pragma unroll
         for (int hh = 0; hh < NHL; ++hh) {
             const int g = g0 + hh;
+            if (ANY && (g >= gq || !in_hd)) continue;   // padding
             const float lsum = h_s[0][g];
             const float* x = v + VPH * hh;
             if (final_out) {
-                store_scaled<VPH>(p.out + (static_cast<int64_t>(b) * p.Hq + h0 + g) * HD + d0, x,
+                store_scaled<VPH>(p.out + (static_cast<int64_t>(b) * p.Hq + h0 + g) * hd + d0, x,
                                   lsum > 0.0f ? 1.0f / lsum : 0.0f);
             } else if constexpr (SPLIT) {  // this wavefront's LDS slot
                 store_scaled<VPH>(&part_acc[wv][g * HD + d0], x, 1.0f);
@@ -615,9 +722,9 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
                     part_ml[wv][1][g] = lsum;
                 }
             } else {  // workspace slot, merged by decode_merge_kernel
-                store_scaled<VPH>(p.ws_acc + (prow * G + g) * HD + d0, x, 1.0f);
+                store_scaled<VPH>(p.ws_acc + (prow * gq + g) * hd + d0, x, 1.0f);
                 if (owns_ml)
-                    *reinterpret_cast<float2*>(p.ws_ml + (prow * G + g) * 2) = make_float2(h_s[1][g], lsum);
+                    *reinterpret_cast<float2*>(p.ws_ml + (prow * gq + g) * 2) = make_float2(h_s[1][g], lsum);
             }
         }
 
@@ -636,9 +743,10 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
         //   out = sum_w acc_w 2^(m_w - M) / sum_w l_w 2^(m_w - M),  M = max_w m_w.
         const int nw = std::min(WPW, cdiv(P_s[b + 1] - P_s[b], NBUF));
         __syncthreads();
-        float* out0 = p.out + (static_cast<int64_t>(b) * p.Hq + h0) * HD;
-        for (int col = threadIdx.x; col < G * HD; col += 64 * WPW) {
-            const int g = col / HD;
+        float* out0 = p.out + (static_cast<int64_t>(b) * p.Hq + h0) * hd;
+        for (int col = threadIdx.x; col < gq * hd; col += 64 * WPW) {
+            const int g = col / hd;
+            const int at = ANY ? g * HD + (col - g * hd) : col;
             float M = -INFINITY;
             for (int u = 0; u < nw; ++u) M = fmaxf(M, part_ml[u][0][g]);
             float L = 0.0f, A = 0.0f;
@@ -646,7 +754,7 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
                 for (int u = 0; u < nw; ++u) {
                     const float wgt = fast_exp2(part_ml[u][0][g] - M);
                     L = fmaf(wgt, part_ml[u][1][g], L);
-                    A = fmaf(wgt, part_acc[u][col], A);
+                    A = fmaf(wgt, part_acc[u][at], A);
                 }
             }
             if (nw > 0) out0[col] = L > 0.0f ? A / L : 0.0f;
@@ -661,7 +769,7 @@ __global__ __launch_bounds__(64 * WPW, mfma_waves_per_simd(HD, G)) void decode_m
 // workgroup), same table preloading, same ring of NBUF blocks per wavefront
 // and the same non-temporal buffer loads, issued in the same order; each
 // consumed block is folded into a wrapping 32-bit sum of its K and V words.
-// sums[b * Hkv + h] receives the sum over the sequence's seq_blocks(b) blocks
+// sums[b * Hkv + h] receives the sum over the sequence's seq_units(b) blocks
 // (all 16 rows of each, the head-h slice of K and of V; a table entry outside
 // the pool contributes 0), so the result checks that every block was read
 // exactly once, whatever the split.  Its time is the rate the decode's
@@ -683,7 +791,7 @@ __global__ __launch_bounds__(64 * WPW) void block_stream_checksum_kernel(DecodeP
     const int w = blockIdx.x * WPW + wv;
     const int kvh = w % Hkv;
     const int range = w / Hkv;
-    const WorkSplit split = build_split(p, P_s, true);
+    const WorkSplit split = build_split<BS>(p, P_s, true);
     if (range >= split.used) return;
     const int64_t row_stride = static_cast<int64_t>(Hkv) * HD;
     const int block_bytes = static_cast<int>(BS * row_stride * 2);
@@ -776,7 +884,7 @@ __global__ __launch_bounds__(64) void decode_generic_kernel(DecodeParams p) {
     const int w = blockIdx.x;
     const int h = w % Hq;
     const int range = w / Hq;
-    const WorkSplit split = build_split(p, P_s, true);
+    const WorkSplit split = build_split<0>(p, P_s, true);
     if (range >= split.used) return;
     const int64_t row_elems = static_cast<int64_t>(p.Hkv) * HD;
     const int range_lo = split.lo(range);
@@ -970,7 +1078,7 @@ __device__ __forceinline__ void merge_few_n(const DecodeParams& p, int grp, int 
 }
 
 __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
-    __shared__ float gm[4], gl[4];
+    __shared__ float gm[4][64], gl[4][64];
     __shared__ float ga[4][64];
     const int t = threadIdx.x;
     const int HD = p.HD, NH = p.NH;
@@ -1009,8 +1117,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
     const int cl = t & 63, pg = t >> 6;
     for (int sub = c0; sub < c1; sub += 64) {
         const int col = sub + cl;
-        // 64 divides HD on the MFMA path; the generic path has one head per segment.
-        const int g = sub / HD;
+        const int g = min(col, c1 - 1) / HD;   // (a slice may span two heads when 64 does not divide HD)
         const int d = min(col, c1 - 1) - g * HD;
         auto row_of = [&](int i) -> int64_t {
             return partial_row(r0 + i, i == 0 && first_tail, p.Hseg, grp) * NH + g;
@@ -1045,20 +1152,18 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(DecodeParams p) {
             }
         }
         __syncthreads();  // the previous sub-pass has read gm, gl, ga
-        if (cl == 0) {
-            gm[pg] = Mt;
-            gl[pg] = Lt;
-        }
+        gm[pg][cl] = Mt;
+        gl[pg][cl] = Lt;
         ga[pg][cl] = At;
         __syncthreads();
         if (pg == 0 && col < c1) {
-            const float M = fmaxf(fmaxf(gm[0], gm[1]), fmaxf(gm[2], gm[3]));
+            const float M = fmaxf(fmaxf(gm[0][cl], gm[1][cl]), fmaxf(gm[2][cl], gm[3][cl]));
             float L = 0.0f, A = 0.0f;
             if (M != -INFINITY) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const float w = fast_exp2(gm[q] - M);
-                    L = fmaf(w, gl[q], L);
+                    const float w = fast_exp2(gm[q][cl] - M);
+                    L = fmaf(w, gl[q][cl], L);
                     A = fmaf(w, ga[q][cl], A);
                 }
             }
@@ -1135,7 +1240,7 @@ bool paired_grid(const DecodeParams& p, int waves, int max_per_simd) {
 // batches and short contexts launch a small grid) and no more than the
 // workspace has partial slots for.
 int decode_ranges(const DecodeParams& p, int waves) {
-    const int64_t max_work = static_cast<int64_t>(p.B) * (p.max_blocks + p.seg_cost);
+    const int64_t max_work = static_cast<int64_t>(p.B) * (p.max_units + p.seg_cost);
     return static_cast<int>(std::max<int64_t>(
         1, std::min<int64_t>({waves / p.Hseg, cdiv<int64_t>(max_work, p.min_per), p.max_slots / p.Hseg})));
 }
@@ -1196,6 +1301,44 @@ int launch_mfma_shape(DecodeParams p, hipStream_t s) {
     return launch_pair(decode_mfma_kernel<HD, G, QF32, 1, NB>, 1, PER_SIMD, p, s, name);
 }
 
+// The ANY instances: head_dim and group padded to the next HD and G.  A short
+// table takes one workgroup per (sequence, kv head) as above where the
+// partials of 8 wavefronts fit LDS (HD <= 128).
+template <int HD, int G>
+int launch_any_shape(DecodeParams p, hipStream_t s) {
+    constexpr int NB = HD == 64 ? 3 : 2;
+    constexpr int PER_SIMD = mfma_waves_per_simd(HD, G);
+    const char* name = "decode_mfma_kernel (any shape)";
+    if (p.bs < 16) {
+        p.seg_cost = kSegmentCost;
+        return launch_pair(decode_mfma_kernel<HD, G, true, 1, NB, false, 2>, 1, PER_SIMD, p, s, name);
+    }
+    if constexpr (HD <= 128) {
+        if (p.max_units <= 8 * 2) {
+            const size_t lds = sizeof(int) * (static_cast<size_t>(p.B) + 1);
+            const unsigned groups = static_cast<unsigned>(p.B) * static_cast<unsigned>(p.Hkv);
+            decode_mfma_kernel<HD, G, true, 8, 2, true, 1><<<groups, 512, lds, s>>>(p);
+            return check_launch(name);
+        }
+    }
+    p.seg_cost = kSegmentCost;
+    if (p.Hkv % 4 == 0)
+        return launch_pair(decode_mfma_kernel<HD, G, true, 4, NB, false, 1>, 4, PER_SIMD, p, s, name);
+    return launch_pair(decode_mfma_kernel<HD, G, true, 1, NB, false, 1>, 1, PER_SIMD, p, s, name);
+}
+
+int launch_any(const DecodeParams& p, hipStream_t s) {
+    const int HD = p.HD <= 64 ? 64 : p.HD <= 128 ? 128 : 256;
+    const int G = p.NH <= 1 ? 1 : p.NH <= 2 ? 2 : p.NH <= 4 ? 4 : p.NH <= 8 ? 8 : 16;
+#define SKV_ANY(HD_, G_) \
+    if (HD == HD_ && G == G_) return launch_any_shape<HD_, G_>(p, s);
+    SKV_ANY(64, 1) SKV_ANY(64, 2) SKV_ANY(64, 4) SKV_ANY(64, 8) SKV_ANY(64, 16)
+    SKV_ANY(128, 1) SKV_ANY(128, 2) SKV_ANY(128, 4) SKV_ANY(128, 8) SKV_ANY(128, 16)
+    SKV_ANY(256, 1) SKV_ANY(256, 2) SKV_ANY(256, 4) SKV_ANY(256, 8) SKV_ANY(256, 16)
+#undef SKV_ANY
+    return set_error(SKV_ERR_UNSUPPORTED, "no decode kernel for head_dim %d, group %d", p.HD, p.NH);
+}
+
 template <bool QF32>
 int launch_mfma(const DecodeParams& p, hipStream_t s) {
     const int G = p.Hq / p.Hkv;
@@ -1249,6 +1392,20 @@ bool mfma_path_ok(const DecodeParams& p, int q_dtype) {
            (q_dtype == SKV_DTYPE_BF16 || q_dtype == SKV_DTYPE_FP32);
 }
 
+// Shapes of the ANY instances.  The bounds are their layouts': 16-byte chunks
+// of rows (head_dim a multiple of 8, aligned pointers), at most 256 dims and
+// 16 query heads per K/V read, units that are whole parts of a block or of
+// whole blocks (a power of two), and the int32 index range of the split in
+// units.  Everything else stays on the generic kernel.
+bool any_path_ok(const DecodeParams& p, int q_dtype) {
+    const int G = p.Hq / p.Hkv;
+    const int64_t units = (static_cast<int64_t>(p.max_blocks) * p.bs + 15) / 16;
+    return (p.bs & (p.bs - 1)) == 0 && p.HD % 8 == 0 && p.HD <= 256 && G <= 16 && aligned16(p.k) && aligned16(p.v) &&
+           aligned16(p.q) && aligned16(p.out) && (q_dtype == SKV_DTYPE_BF16 || q_dtype == SKV_DTYPE_FP32) &&
+           p.B * (units + kSegmentCost) < (int64_t{1} << 30) && static_cast<int64_t>(p.max_blocks) * p.bs <= INT32_MAX &&
+           static_cast<int64_t>(p.Hkv) * p.HD <= (1 << 24);
+}
+
 // The appended rows go through the MFMA kernel when it runs and its 16-byte
 // accesses to them are aligned; otherwise the append kernel runs first (same
 // result: it writes position lens[b] - 1 of every sequence, then the decode
@@ -1265,14 +1422,21 @@ int run_decode_chunk(DecodeParams p, int q_dtype, char* ws, const WorkspaceLayou
     p.ws_ml = reinterpret_cast<float*>(ws + w.ml_off);
     p.ws_acc = reinterpret_cast<float*>(ws + w.acc_off);
     const bool mfma = mfma_path_ok(p, q_dtype);
-    if (p.k_new != nullptr && !(mfma && aligned16(p.k_new) && aligned16(p.v_new)))
+    const bool any = !mfma && any_path_ok(p, q_dtype);
+    if (p.k_new != nullptr && !((mfma || any) && aligned16(p.k_new) && aligned16(p.v_new)))
         if (int rc = append_before_decode(p, s)) return rc;
-    if (mfma) {
+    if (mfma || any) {
         p.Hseg = p.Hkv;
         p.NH = p.Hq / p.Hkv;
         p.min_per = 4;
+        p.max_units = mfma ? p.max_blocks : static_cast<int>((static_cast<int64_t>(p.max_blocks) * p.bs + 15) / 16);
+        p.max_tokens = any ? p.max_blocks * p.bs : 0;
+        p.bs_log2 = __builtin_ctz(p.bs);
+        p.q_fp32 = q_dtype == SKV_DTYPE_FP32 ? 1 : 0;
+        if (any) return launch_any(p, s);
         return q_dtype == SKV_DTYPE_FP32 ? launch_mfma<true>(p, s) : launch_mfma<false>(p, s);
     }
+    p.max_units = p.max_blocks;
     p.Hseg = p.Hq;
     p.NH = 1;
     p.min_per = std::max(1, cdiv(64, p.bs));
@@ -1601,6 +1765,7 @@ extern "C" int skv_paged_block_checksum(const uint16_t* k_pool, const uint16_t* 
     p.Hseg = num_kv_heads;
     p.NH = num_q_heads / num_kv_heads;
     p.min_per = 4;
+    p.max_units = max_blocks_per_seq;
     p.max_slots = kMaxWaves;
     if (!mfma_path_ok(p, SKV_DTYPE_BF16) || !aligned16(k_pool) || !aligned16(v_pool))
         return set_error(SKV_ERR_UNSUPPORTED,

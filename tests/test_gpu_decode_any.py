@@ -1,0 +1,103 @@
+"""Decode shapes outside the tuned geometry (any group up to 16, head_dim in multiples of 8 up to 256,
+power-of-two block sizes) and the ones just past those bounds, against the oracle in float64: the plain
+call and the fused append, short and long tables, cut blocks, absent entries, NaN in unused slots."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from kvcase import make_case
+
+pytestmark = pytest.mark.gpu
+
+# Scores of N(0,1) rows are below ~2^5 in log2 units, so an fp32 score is off by at most a few 2^-19 and a
+# probability by the same relative amount; sums of fp32 products add less.  Queries are exact.
+REL = 8e-6
+
+# (Hq, Hkv, hd, block size)
+SHAPES = [(24, 8, 128, 16), (5, 1, 64, 16), (28, 4, 128, 16), (13, 1, 128, 16), (40, 8, 128, 16), (9, 3, 64, 16),
+          (8, 2, 96, 16), (8, 2, 40, 16), (8, 1, 256, 16), (6, 2, 200, 16), (32, 2, 256, 16), (3, 3, 8, 16),
+          (16, 4, 128, 32), (12, 4, 64, 64), (8, 8, 128, 1024), (32, 4, 64, 8), (8, 2, 128, 4), (15, 1, 256, 2),
+          (32, 4, 64, 1), (6, 2, 96, 8),
+          # past the bounds: the generic kernel
+          (34, 2, 64, 16), (6, 3, 40, 5), (8, 2, 264, 16), (4, 2, 36, 16), (8, 2, 64, 48)]
+LENS = {"short": [1, 17, 40, 0, 256, 129], "long": [1, 70, 2049, 0, 513, 260, 3000], "one": [9001]}
+
+
+def _run(skv, c, append, kv_fp32, k_new, v_new):
+    d = {n: skv.DeviceBuffer.from_numpy(c[n]) for n in ("q_dev", "k_pool", "v_pool", "tables", "lens")}
+    shape = (c["B"], c["Hq"], c["hd"])
+    out = skv.DeviceBuffer.from_numpy(np.full(shape, np.nan, np.float32))
+    ws, wsb = skv.decode_workspace(c["B"], c["Hq"], c["Hkv"], c["hd"])
+    qd = skv.DTYPE_BF16 if c["q_dtype"] == "bf16" else skv.DTYPE_FP32
+    tail = (d["lens"], c["B"], c["Hq"], c["Hkv"], c["hd"], c["bs"], c["scale"], out, ws, wsb)
+    if append:
+        dk, dv = skv.DeviceBuffer.from_numpy(k_new), skv.DeviceBuffer.from_numpy(v_new)
+        skv.paged_decode_append(d["q_dev"], qd, dk, dv, skv.DTYPE_FP32 if kv_fp32 else skv.DTYPE_BF16, d["k_pool"],
+                                d["v_pool"], c["total_blocks"], d["tables"], c["tables"].shape[1], *tail)
+    else:
+        skv.paged_decode(d["q_dev"], qd, d["k_pool"], d["v_pool"], c["total_blocks"], d["tables"], c["tables"].shape[1],
+                         *tail)
+    skv.synchronize()
+    return (out.download(np.float32, shape), d["k_pool"].download(np.uint16, c["k_pool"].shape),
+            d["v_pool"].download(np.uint16, c["v_pool"].shape))
+
+
+def _reference(c):
+    """float64 attention over the positions whose table entry exists."""
+    out = np.zeros((c["B"], c["Hq"], c["hd"]))
+    G, bs = c["Hq"] // c["Hkv"], c["bs"]
+    for b, L in enumerate(c["lens"]):
+        pos = np.arange(min(int(L), c["tables"].shape[1] * bs))
+        ids = c["tables"][b, pos // bs]
+        ok = (ids >= 0) & (ids < c["total_blocks"])
+        if not ok.any():
+            continue
+        k = oracle.bf16_to_f32(c["k_pool"][ids[ok], pos[ok] % bs]).astype(np.float64)
+        v = oracle.bf16_to_f32(c["v_pool"][ids[ok], pos[ok] % bs]).astype(np.float64)
+        for h in range(c["Hq"]):
+            s = k[:, h // G] @ c["q_ref"][b, h].astype(np.float64) * c["scale"]
+            w = np.exp(s - s.max())
+            out[b, h] = w @ v[:, h // G] / w.sum()
+    return out
+
+
+@pytest.mark.parametrize("lens", list(LENS))
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "-".join(map(str, s)))
+def test_any_shape(gpu, shape, lens):
+    Hq, Hkv, hd, bs = shape
+    ctx = LENS[lens]
+    seed = Hq * 1000 + hd + bs + len(ctx)
+    rng = np.random.default_rng(seed)
+    q_dtype = "fp32" if (Hq + hd + len(ctx)) % 2 else "bf16"
+    c = make_case(len(ctx), Hq, Hkv, hd, bs, ctx, layout="random", q_dtype=q_dtype, seed=seed,
+                  extra_cols=0 if lens == "short" else 2)
+    if len(ctx) > 1:  # a hole in the middle of one sequence, an id past the pool in another
+        c["tables"][-1, 0] = -1
+        c["tables"][2, 40 // bs // 2] = c["total_blocks"] + 3
+    for b, L in enumerate(ctx):  # slots past the context hold NaN
+        if 0 < L and L % bs and 0 <= c["tables"][b, L // bs] < c["total_blocks"]:
+            c["k_pool"][c["tables"][b, L // bs], L % bs:] = 0x7FC0
+            c["v_pool"][c["tables"][b, L // bs], L % bs:] = 0x7FC0
+    for append in (False, True):
+        kv_fp32 = append and hd % 16 == 0
+        new = rng.standard_normal((2, len(ctx), Hkv * hd), dtype=np.float32)
+        bits = oracle.f32_to_bf16(new)
+        k_new, v_new = new if kv_fp32 else bits
+        if not append:
+            ref_c = c
+        else:
+            ref_c = dict(c, k_pool=c["k_pool"].copy(), v_pool=c["v_pool"].copy())
+            for b, L in enumerate(ctx):
+                e = c["tables"][b, (L - 1) // bs] if L > 0 else -1
+                if 0 <= e < c["total_blocks"]:
+                    ref_c["k_pool"][e, (L - 1) % bs] = bits[0, b].reshape(Hkv, hd)
+                    ref_c["v_pool"][e, (L - 1) % bs] = bits[1, b].reshape(Hkv, hd)
+        got, gk, gv = _run(gpu, c, append, kv_fp32, k_new, v_new)
+        np.testing.assert_array_equal(gk, ref_c["k_pool"])
+        np.testing.assert_array_equal(gv, ref_c["v_pool"])
+        ref = _reference(ref_c)
+        assert np.isfinite(got).all()
+        rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert rel <= REL, f"append={append} q={q_dtype}: relative error {rel:.2e}"
