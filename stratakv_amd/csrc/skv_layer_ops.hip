@@ -348,11 +348,37 @@ const RopeTable& rope_inv_freq(int hd) {
 
 // cos and sin of position * inv (angle in double, rounded to float): the
 // values rope_table computes on the host, for kernels that rotate several
-// positions.
+// positions.  The angle (below 2^31) is reduced by multiples of pi/2 held in
+// two doubles and the Taylor series of both functions to degree 16 / 17 on
+// [-pi/4, pi/4] are summed in double (truncation below 2^-56, rounding below
+// 2^-52): the float results are those of correctly rounded double functions
+// but for a tie within 2^-52.  The general sin and cos of double took ~4 us a
+// projection of rotated outputs.
 __device__ __forceinline__ void rope_cos_sin(int position, float inv, float& c, float& s) {
     const double angle = static_cast<double>(position) * static_cast<double>(inv);
-    c = static_cast<float>(cos(angle));
-    s = static_cast<float>(sin(angle));
+    const double n = rint(angle * 0.63661977236758134308);
+    const double r = fma(-n, 6.12323399573676603587e-17, fma(-n, 1.57079632679489655800, angle));
+    const double z = r * r;
+    double ps = 1.0 / 355687428096000.0, pc = 1.0 / 20922789888000.0;
+    ps = fma(ps, z, -1.0 / 1307674368000.0);
+    ps = fma(ps, z, 1.0 / 6227020800.0);
+    ps = fma(ps, z, -1.0 / 39916800.0);
+    ps = fma(ps, z, 1.0 / 362880.0);
+    ps = fma(ps, z, -1.0 / 5040.0);
+    ps = fma(ps, z, 1.0 / 120.0);
+    ps = fma(ps, z, -1.0 / 6.0);
+    const float sn = static_cast<float>(fma(r * z, ps, r));
+    pc = fma(pc, z, -1.0 / 87178291200.0);
+    pc = fma(pc, z, 1.0 / 479001600.0);
+    pc = fma(pc, z, -1.0 / 3628800.0);
+    pc = fma(pc, z, 1.0 / 40320.0);
+    pc = fma(pc, z, -1.0 / 720.0);
+    pc = fma(pc, z, 1.0 / 24.0);
+    pc = fma(pc, z, -0.5);
+    const float cn = static_cast<float>(fma(pc, z, 1.0));
+    const int q = static_cast<int>(static_cast<int64_t>(n) & 3);
+    c = q == 0 ? cn : q == 1 ? -sn : q == 2 ? -cn : sn;
+    s = q == 0 ? sn : q == 1 ? cn : q == 2 ? -sn : -cn;
 }
 
 __device__ __forceinline__ float swiglu_of(float g, float u) {
@@ -811,16 +837,13 @@ int launch_fused_rows(const FusedGemv& f, bool bf16, int items, hipStream_t s) {
 typedef __bf16 mm_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t mm_u32x4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kMmTokens = 64;                      // tokens per workgroup (4 column tiles of 16)
-constexpr int kMmWaves = 4;                        // wavefronts per workgroup, one feature group each
-constexpr int kMmStageK = 64;                      // k per LDS stage (two 32-wide MFMA steps)
-constexpr int kMmRowBytes = kMmStageK * 2 + 16;    // one token's stage in LDS (bf16, padded)
-constexpr int kMmRing = 2;                         // stages of operands in flight
+constexpr int kMmWaves = 8;      // wavefronts per workgroup
+constexpr int kMmStageK = 32;    // k per stage and K part: one MFMA step
 
 struct MmArgs {
     FusedGemv f;
     int groups;                 // 32-feature groups
-    int token_tiles;            // cdiv(rows, kMmTokens)
+    int token_tiles;            // cdiv(rows, tokens per workgroup)
 };
 
 // Feature group `g` (32 outputs as two 16-row tiles) of a projection:
@@ -856,205 +879,328 @@ __device__ __forceinline__ MmGroup mm_group(const FusedGemv& f, int g) {
     return q;
 }
 
-// One workgroup = kMmWaves / KS feature groups x kMmTokens tokens, K split
-// into KS parts (KS = 2 when the grid would be too small to fill the chip):
-// wavefront w computes group w % (kMmWaves / KS) over part w / (kMmWaves / KS)
-// and the parts are summed through LDS in a fixed order.  The inputs go
-// through LDS in stages of kMmStageK per part: each thread loads 16
-// consecutive fp32 of one token per part, splits them into hi and lo parts
-// and stores them (two LDS buffers, one barrier per stage); a wavefront reads
-// them in the MFMA B layout (lane (t, j): token t of a column tile, k chunk
-// 8j..8j+7) and its weight rows straight from global memory in the A layout
-// (row t of a tile, the same chunk).  Inputs and weights are requested
-// kMmRing stages ahead, the inputs of a stage after its weights, so that each
-// wait in issue order covers exactly the stage it needs.  Output lane layout:
-// acc[a][c][i] = feature (tile a) 4j + i, token 16c + t.
-constexpr int kMmPartBytes = 2 * kMmTokens * kMmRowBytes;   // hi + lo of one part's stage
+typedef __bf16 pg_bf16x2_t __attribute__((ext_vector_type(2)));
 
-template <int MODE, int KS>
-__global__ __launch_bounds__(64 * kMmWaves) void proj_mm_kernel(MmArgs args) {
-    constexpr int GPW = kMmWaves / KS;   // feature groups per workgroup
+// hi = bf16(v) (round to nearest even) of two values and lo = bf16 of the
+// exact remainders v - hi, packed two to a word.
+__device__ __forceinline__ void split_pair(float v0, float v1, uint32_t& hi, uint32_t& lo) {
+    const pg_bf16x2_t h = {static_cast<__bf16>(v0), static_cast<__bf16>(v1)};
+    hi = __builtin_bit_cast(uint32_t, h);
+    const pg_bf16x2_t l = {static_cast<__bf16>(v0 - bf16_lo(hi)), static_cast<__bf16>(v1 - bf16_hi(hi))};
+    lo = __builtin_bit_cast(uint32_t, l);
+}
+
+// Four fp32 values as PARTS bf16 parts, two to a word.  2: hi = bf16(v) (round
+// to nearest even) and lo = bf16 of the exact remainder, the split of the
+// prompt projections.  3: the exact split of split3_pair, for skv_linear_f32,
+// whose inputs keep all 24 bits.
+template <int PARTS>
+__device__ __forceinline__ void mm_split4(const f32x4_t& v, uint2 (&w)[PARTS]) {
+    if constexpr (PARTS == 2) {
+        split_pair(v[0], v[1], w[0].x, w[1].x);
+        split_pair(v[2], v[3], w[0].y, w[1].y);
+    } else {
+        uint32_t a[3], b[3];
+        split3_pair(v[0], v[1], a);
+        split3_pair(v[2], v[3], b);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) w[i] = make_uint2(a[i], b[i]);
+    }
+}
+
+// Bias, RoPE, SwiGLU or residual and the stores of features 4j .. 4j+3 of a
+// group's two tiles (sums `a`, `b`) for token `tok`.
+template <int MODE>
+__device__ __forceinline__ void mm_finish(const FusedGemv& f, const MmGroup& grp, const f32x4_t& a, const f32x4_t& b,
+                                          int tok, int j) {
+    if (tok >= f.rows) return;
+    auto bias4 = [&](int m, int r) {
+        const float* p = pick3(f.bias, m);
+        return p != nullptr ? f32x4_t{p[r], p[r + 1], p[r + 2], p[r + 3]} : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    const int ra = grp.r0 + 4 * j, rb = grp.r1 + 4 * j;
+    if constexpr (MODE == FUSED_QKV) {
+        f32x4_t ya = a + bias4(grp.m, ra), yb = b + bias4(grp.m, rb);
+        if (grp.rope) {
+            const int half = f.head_dim / 2;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float cs, sn, va = ya[i], vb = yb[i];
+                rope_cos_sin(f.position + tok, f.rope.cs[(ra + i) % f.head_dim % half], cs, sn);
+                rotate_pair(va, vb, cs, sn);
+                ya[i] = va;
+                yb[i] = vb;
+            }
+        }
+        float* y = pick3(f.y, grp.m) + static_cast<int64_t>(tok) * pick3(f.n, grp.m);
+        *reinterpret_cast<f32x4_t*>(y + ra) = ya;
+        *reinterpret_cast<f32x4_t*>(y + rb) = yb;
+    } else if constexpr (MODE == FUSED_GATE_UP) {
+        const f32x4_t gv = a + bias4(0, ra), uv = b + bias4(1, ra);
+        const f32x4_t act = {swiglu_of(gv[0], uv[0]), swiglu_of(gv[1], uv[1]), swiglu_of(gv[2], uv[2]),
+                             swiglu_of(gv[3], uv[3])};
+        *reinterpret_cast<f32x4_t*>(f.y[0] + static_cast<int64_t>(tok) * f.n[0] + ra) = act;
+    } else {
+        const int64_t row = static_cast<int64_t>(tok) * f.n[0];
+        f32x4_t ya = a + bias4(0, ra), yb = b + bias4(0, rb);
+        if constexpr (MODE == FUSED_RESIDUAL) {
+            ya += *reinterpret_cast<const f32x4_t*>(f.residual + row + ra);
+            yb += *reinterpret_cast<const f32x4_t*>(f.residual + row + rb);
+        }
+        *reinterpret_cast<f32x4_t*>(f.y[0] + row + ra) = ya;
+        *reinterpret_cast<f32x4_t*>(f.y[0] + row + rb) = yb;
+    }
+}
+
+// One workgroup = 8 wavefronts = WF x WT x KS over a tile of WF * FG feature
+// groups (32 features each) and 16 WT * CT tokens: a wavefront computes FG
+// groups x CT column tiles over one of KS parts of K, and the parts are summed
+// through LDS in a fixed order.  K goes in stages of 32 per part through two LDS
+// buffers, one barrier per stage: every thread loads 16-byte pieces of the bf16
+// weight rows and of the fp32 token rows, consecutive lanes on consecutive
+// bytes, splits the latter and stores both; the wavefronts read both operands
+// in the MFMA layouts (lane (t, j): row or token t, k chunk 8j..8j+7).  Output
+// lane layout: acc[a][c][i] = feature (tile a) 4j + i, token 16c + t.
+//
+// What bounds it at prompt lengths of tens to hundreds of tokens is feeding the
+// CUs, not the products:
+// * Weights read straight into the A layout, as before, put neighbouring lanes
+//   on different rows, ~90 clocks of the CU's address unit per wave-wide load
+//   whether the line is in L2 or not; through LDS a load covers whole lines.
+// * Loads return in issue order, so the inputs of the next stage, which must be
+//   in registers to be stored, hold back nothing only if they were requested as
+//   early as its weights: both go through a register ring of RING stages.
+// * K is split over the wavefronts of a workgroup, not over workgroups: the
+//   entry points have no scratch to add partial sums in.
+template <int PARTS, int WF, int FG, int WT, int CT, int KS, int RING>
+struct MmShape {
+    static constexpr int kGroups = WF * FG, kTokens = 16 * WT * CT;
+    static constexpr int RB = kMmStageK * 2;   // LDS row of a stage (bf16), 4 chunks of 16 bytes
+    // Byte offset of 16-byte chunk c of row r: XOR-swizzled so that the operand
+    // reads are free of bank conflicts.  (Rows padded by 16 bytes had the LDS
+    // busy 92k of 130k cycles, half of them conflicts: a wave-wide 16-byte read
+    // serves lanes 0-3, 12-15 and 20-27 together, not 16 consecutive ones.)
+    __host__ __device__ static constexpr int at(int r, int c) {
+        return r * RB + (c ^ ((r >> 2) & 2)) * 16;
+    }
+    static constexpr int kPartBytes = (32 * kGroups + PARTS * kTokens) * RB;   // one K part's stage: weights, input parts
+    static constexpr int kSumBytes = KS > 1 ? kMmWaves * 2 * FG * CT * 1024 : 0;
+    static constexpr int kLds = 2 * KS * kPartBytes > kSumBytes ? 2 * KS * kPartBytes : kSumBytes;
+    static_assert(WF * WT * KS == kMmWaves, "wavefronts");
+    static_assert(kLds <= 160 * 1024, "LDS");
+};
+
+template <int MODE, int PARTS, int WF, int FG, int WT, int CT, int KS, int RING>
+__global__ __launch_bounds__(64 * kMmWaves, 2) void proj_mm_kernel(MmArgs args) {
+    using Shape = MmShape<PARTS, WF, FG, WT, CT, KS, RING>;
+    constexpr int SK = kMmStageK;
+    constexpr int NT = Shape::kTokens, NG = Shape::kGroups;
+    constexpr int TPP = 64 * kMmWaves / KS;            // threads staging one K part
+    constexpr int CW = SK / 8, CX = SK / 4;            // 16-byte pieces per weight row and per token row
+    constexpr int WL = 32 * NG * CW / TPP, XL = NT * CX / TPP;   // pieces per thread and stage
+    static_assert(WL * TPP == 32 * NG * CW && XL * TPP == NT * CX, "staging split");
     const FusedGemv& f = args.f;
-    extern __shared__ __align__(16) unsigned char xs[];   // [buffer][part][hi, lo][token]
-    auto xs_at = [&](int buf, int part, int half) { return xs + ((buf * KS + part) * 2 + half) * (kMmPartBytes / 2); };
+    extern __shared__ __align__(16) unsigned char xs[];   // [buffer][K part][weight rows, then input parts x tokens]
+    auto w_at = [&](int buf, int part) { return xs + (buf * KS + part) * Shape::kPartBytes; };
+    auto x_at = [&](int buf, int part, int h) { return w_at(buf, part) + (32 * NG + h * NT) * Shape::RB; };
     const int tid = threadIdx.x, lane = tid & 63, t = lane & 15, j = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int part = w / GPW;
+    const int part = w / (WF * WT), wf = w / WT % WF, wt = w % WT;
     // Workgroups are dealt to the 8 XCDs round-robin: the token tiles of one
     // feature tile go to the same XCD, one after another, so its weight rows
     // are read from HBM once and then from that XCD's L2.
     const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
     const int ftile = (local / args.token_tiles) * 8 + xcd;
-    const int tile = local % args.token_tiles;
-    if (ftile * GPW >= args.groups) return;      // the whole workgroup, before any barrier
-    const int g = ftile * GPW + w % GPW;
-    const bool live = g < args.groups;           // a wave past the last group stores nothing
-    const MmGroup grp = mm_group<MODE>(f, min(g, args.groups - 1));
-    const int K = f.K, rows = f.rows, nst = K / kMmStageK / KS;   // stages per part
-    const int tok0 = tile * kMmTokens;
+    const int tok0 = local % args.token_tiles * NT;
+    if (ftile * NG >= args.groups) return;       // the whole workgroup, before any barrier
+    const int K = f.K, rows = f.rows;
+    // Stages of part q: [first(q), first(q + 1)), as even as K / SK allows
+    // (`each` or one more).
+    const int total = K / SK, each = total / KS, more = total % KS;
+    auto first = [&](int q) { return q * each + min(q, more); };
+    const int s_count = first(part + 1) - first(part);
 
-    // Staging: thread -> token tid / 4, k (tid % 4) * 16 .. + 15 of a stage.
-    const int st_tok = tid >> 2, st_k = (tid & 3) * 16;
-    const float* xrow = f.x + static_cast<int64_t>(min(tok0 + st_tok, rows - 1)) * K + st_k;
-    // Weight rows of this wavefront's two tiles.
-    const int mb = MODE == FUSED_GATE_UP ? 1 : grp.m;
-    const char* wa = static_cast<const char*>(f.w[grp.m]) + static_cast<int64_t>(grp.r0 + t) * f.row_bytes[grp.m];
-    const char* wb = static_cast<const char*>(f.w[mb]) + static_cast<int64_t>(grp.r1 + t) * f.row_bytes[mb];
-
+    // Staging: thread -> K part tid / TPP; groups and tokens past the end repeat the last one.
+    const int st_part = tid / TPP, u0 = tid % TPP;
+    const int st_first = first(st_part);
+    const char* wrow[WL];
+    const float* xrow[XL];
+    int w_off[WL], x_off[XL];   // byte offsets in LDS
+#pragma unroll
+    for (int i = 0; i < WL; ++i) {
+        const int u = u0 + i * TPP, row = u / CW;
+        const MmGroup grp = mm_group<MODE>(f, min(ftile * NG + row / 32, args.groups - 1));
+        const int second = row / 16 % 2;
+        const int m = MODE == FUSED_GATE_UP ? second : grp.m;
+        wrow[i] = static_cast<const char*>(pick3(f.w, m)) +
+                  static_cast<int64_t>((second ? grp.r1 : grp.r0) + row % 16) * pick3(f.row_bytes, m) + u % CW * 16;
+        w_off[i] = Shape::at(row, u % CW);
+    }
+#pragma unroll
+    for (int i = 0; i < XL; ++i) {
+        const int u = u0 + i * TPP, row = u / CX;
+        xrow[i] = f.x + static_cast<int64_t>(min(tok0 + row, rows - 1)) * K + u % CX * 4;
+        x_off[i] = Shape::at(row, u % CX / 2) + u % CX % 2 * 8;
+    }
     struct Stage {
-        mm_u32x4_t wop[2][2];   // [k-step][tile] weight operands of this wavefront's part
-        f32x4_t x[KS][4];       // this thread's 16 staged inputs of every part
+        mm_u32x4_t w[WL];
+        f32x4_t x[XL];
     };
-    auto load = [&](int s, Stage& o) __attribute__((always_inline)) {
-        s = min(s, nst - 1);    // past the end: the last stage again (in bounds, unused)
+    auto load = [&](int s, Stage& o) __attribute__((always_inline)) {   // past the end: the last stage again (unused)
+        const int at = min(st_first + s, total - 1) * SK;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int k = (part * nst + s) * kMmStageK + ks * 32 + 8 * j;
-            o.wop[ks][0] = *reinterpret_cast<const mm_u32x4_t*>(wa + 2 * k);
-            o.wop[ks][1] = *reinterpret_cast<const mm_u32x4_t*>(wb + 2 * k);
-        }
+        for (int i = 0; i < WL; ++i) o.w[i] = *reinterpret_cast<const mm_u32x4_t*>(wrow[i] + 2 * at);
 #pragma unroll
-        for (int q = 0; q < KS; ++q)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                o.x[q][r] = reinterpret_cast<const f32x4_t*>(xrow + (q * nst + s) * kMmStageK)[r];
+        for (int i = 0; i < XL; ++i) o.x[i] = *reinterpret_cast<const f32x4_t*>(xrow[i] + at);
     };
-    auto stage_inputs = [&](int buf, const Stage& o) __attribute__((always_inline)) {
+    auto stage = [&](int buf, const Stage& o) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < KS; ++q) {
-            // hi = bf16(v) for a pair in one conversion; its two values back as
-            // floats with a byte permute (low half to the top) and a mask; lo =
-            // bf16 of the exact remainder v - hi, one conversion per pair.
-            typedef __bf16 mm_bf16x2_t __attribute__((ext_vector_type(2)));
-            uint32_t hw[8], lw[8];
+        for (int i = 0; i < WL; ++i) *reinterpret_cast<mm_u32x4_t*>(w_at(buf, st_part) + w_off[i]) = o.w[i];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float v0 = o.x[q][e >> 1][2 * (e & 1)], v1 = o.x[q][e >> 1][2 * (e & 1) + 1];
-                const mm_bf16x2_t h = {static_cast<__bf16>(v0), static_cast<__bf16>(v1)};
-                hw[e] = __builtin_bit_cast(uint32_t, h);
-                const float h0 = __uint_as_float(__builtin_amdgcn_perm(hw[e], hw[e], 0x01000c0cu));
-                const float h1 = __uint_as_float(hw[e] & 0xFFFF0000u);
-                const mm_bf16x2_t l = {static_cast<__bf16>(v0 - h0), static_cast<__bf16>(v1 - h1)};
-                lw[e] = __builtin_bit_cast(uint32_t, l);
-            }
-            unsigned char* dh = xs_at(buf, q, 0) + st_tok * kMmRowBytes + st_k * 2;
-            unsigned char* dl = xs_at(buf, q, 1) + st_tok * kMmRowBytes + st_k * 2;
-            reinterpret_cast<mm_u32x4_t*>(dh)[0] = mm_u32x4_t{hw[0], hw[1], hw[2], hw[3]};
-            reinterpret_cast<mm_u32x4_t*>(dh)[1] = mm_u32x4_t{hw[4], hw[5], hw[6], hw[7]};
-            reinterpret_cast<mm_u32x4_t*>(dl)[0] = mm_u32x4_t{lw[0], lw[1], lw[2], lw[3]};
-            reinterpret_cast<mm_u32x4_t*>(dl)[1] = mm_u32x4_t{lw[4], lw[5], lw[6], lw[7]};
+        for (int i = 0; i < XL; ++i) {
+            uint2 p[PARTS];
+            mm_split4<PARTS>(o.x[i], p);
+#pragma unroll
+            for (int h = 0; h < PARTS; ++h) *reinterpret_cast<uint2*>(x_at(buf, st_part, h) + x_off[i]) = p[h];
         }
     };
 
-    f32x4_t acc[2][4];
+    // PARTS 3 sums in two levels: `acc` over 64 k (192 products of parts), then
+    // into `sum`.  One chain over K rounds every addition at the size of the
+    // whole sum and was twice as far from float64 as the one-row kernel, whose
+    // 64 lanes sum 64 short chains (K 14,336: 6.6e-7 against 3.1e-7 of the
+    // products' norm).
+    f32x4_t acc[2 * FG][CT], sum[2 * FG][CT];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < 2 * FG; ++a)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[a][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    auto compute = [&](int buf, const Stage& o) __attribute__((always_inline)) {
+        for (int c = 0; c < CT; ++c) acc[a][c] = sum[a][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    auto flush = [&]() __attribute__((always_inline)) {
+        if constexpr (PARTS == 3) {
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            mm_u32x4_t bh[4], bl[4];
+            for (int a = 0; a < 2 * FG; ++a)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int off = (16 * c + t) * kMmRowBytes + (ks * 32 + 8 * j) * 2;
-                bh[c] = *reinterpret_cast<const mm_u32x4_t*>(xs_at(buf, part, 0) + off);
-                bl[c] = *reinterpret_cast<const mm_u32x4_t*>(xs_at(buf, part, 1) + off);
-            }
-            // All hi products, then all lo products: no MFMA waits on the one
-            // issued just before it.
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(mm_bf16x8_t, o.wop[ks][a]), __builtin_bit_cast(mm_bf16x8_t, bh[c]),
-                        acc[a][c], 0, 0, 0);
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(mm_bf16x8_t, o.wop[ks][a]), __builtin_bit_cast(mm_bf16x8_t, bl[c]),
-                        acc[a][c], 0, 0, 0);
+                for (int c = 0; c < CT; ++c) {
+                    sum[a][c] += acc[a][c];
+                    acc[a][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                }
         }
     };
-
-    // Ring: slot u holds stage s0 + u (weights for the compute of that stage,
-    // inputs for its staging one stage earlier).  Stage 0's inputs are staged
-    // before the loop; the loop computes stage s, then stages s + 1.
-    Stage ring[kMmRing];
+    struct Ops {
+        mm_u32x4_t a[2 * FG], b[PARTS][CT];
+    };
+    auto read_ops = [&](int buf, Ops& o) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kMmRing; ++u) load(u, ring[u]);
-    stage_inputs(0, ring[0]);
+        for (int a = 0; a < 2 * FG; ++a)
+            o.a[a] = *reinterpret_cast<const mm_u32x4_t*>(w_at(buf, part) + Shape::at((wf * 2 * FG + a) * 16 + t, j));
+#pragma unroll
+        for (int h = PARTS - 1; h >= 0; --h)
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+                o.b[h][c] = *reinterpret_cast<const mm_u32x4_t*>(x_at(buf, part, h) + Shape::at((wt * CT + c) * 16 + t, j));
+    };
+    // Smallest parts first; no MFMA waits on the one issued just before it.
+    auto multiply = [&](const Ops& o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = PARTS - 1; h >= 0; --h)
+#pragma unroll
+            for (int a = 0; a < 2 * FG; ++a)
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+                    acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mm_bf16x8_t, o.a[a]),
+                                                                        __builtin_bit_cast(mm_bf16x8_t, o.b[h][c]),
+                                                                        acc[a][c], 0, 0, 0);
+    };
+
+    // Iteration s multiplies stage s, whose operands are in registers, reads
+    // the operands of stage s + 1 from LDS, splits and stores stage s + 2 into
+    // the buffer stage s came from, and requests stage s + 2 + RING into the
+    // ring slot that freed: nothing in it depends on anything else in it, and
+    // the products are interleaved with the rest, so the matrix, vector and LDS
+    // units work side by side between two barriers.  Whole rounds of the ring
+    // run with nothing conditional (a branch makes the compiler's wait counts
+    // after it assume the worst and wait for the whole ring), then the rest.
+    Stage ring[RING];
+    Ops ops[2];
+    {
+        Stage s0, s1;
+        load(0, s0);
+        load(1, s1);
+#pragma unroll
+        for (int u = 0; u < RING; ++u) load(2 + u, ring[u]);
+        stage(0, s0);
+        stage(1, s1);
+    }
     __syncthreads();
-    for (int s0 = 0; s0 < nst; s0 += kMmRing) {   // nst is a multiple of kMmRing
+    read_ops(0, ops[0]);
+    __syncthreads();   // stage 0's buffer is free
+    auto iterate = [&](int s, int u, bool multiplies) __attribute__((always_inline)) {
+        read_ops((s + 1) & 1, ops[(u + 1) & 1]);
+        stage(s & 1, ring[u]);
+        load(s + 2 + RING, ring[u]);
+        if (multiplies) multiply(ops[u & 1]);
+        if (u % 2 == 1) flush();
+    };
+    static_assert(RING % 2 == 0, "operand registers, sums of 64 k");
+    const int rounds = each / RING * RING;
+    for (int s0 = 0; s0 < rounds; s0 += RING) {
 #pragma unroll
-        for (int u = 0; u < kMmRing; ++u) {
-            const int s = s0 + u;
-            compute(s & 1, ring[u]);
-            load(s + kMmRing, ring[u]);
-            __builtin_amdgcn_sched_barrier(0);   // issue order kept: the loads stay kMmRing stages ahead
-            stage_inputs((s + 1) & 1, ring[(u + 1) % kMmRing]);
+        for (int u = 0; u < RING; ++u) {
+            iterate(s0 + u, u, true);
+#pragma unroll
+            for (int i = 0; i < PARTS * 2 * FG * CT; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // VALU
+                __builtin_amdgcn_sched_group_barrier(0x080, 1, 0);   // DS
+            }
             __syncthreads();
         }
     }
-    if constexpr (KS == 2) {
-        // Part 1's sums into LDS (the staging buffers are idle after the
-        // last barrier), then part 0 adds them: part 0 + part 1.
-        f32x4_t* red = reinterpret_cast<f32x4_t*>(xs) + (w % GPW) * 8 * 64;
-        if (part == 1) {
+    const int nst = each + (more > 0 ? 1 : 0);
 #pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) red[(4 * a + c) * 64 + lane] = acc[a][c];
+    for (int u = 0; u < RING; ++u) {
+        if (rounds + u < nst) {   // workgroup-uniform
+            iterate(rounds + u, u, rounds + u < s_count);
+            __syncthreads();
         }
-        __syncthreads();
-        if (part == 1) return;
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[a][c] += red[(4 * a + c) * 64 + lane];
     }
-    if (!live) return;
-
-    auto bias4 = [&](int m, int r) {
-        const float* b = f.bias[m];
-        return b != nullptr ? f32x4_t{b[r], b[r + 1], b[r + 2], b[r + 3]} : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    };
+    if constexpr (PARTS == 3) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int tok = tok0 + 16 * c + t;
-        if (tok >= rows) continue;
-        const int ra = grp.r0 + 4 * j, rb = grp.r1 + 4 * j;
-        if constexpr (MODE == FUSED_QKV) {
-            f32x4_t ya = acc[0][c] + bias4(grp.m, ra), yb = acc[1][c] + bias4(grp.m, rb);
-            if (grp.rope) {
-                const int half = f.head_dim / 2;
+        for (int a = 0; a < 2 * FG; ++a)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float cs, sn, va = ya[i], vb = yb[i];
-                    rope_cos_sin(f.position + tok, f.rope.cs[(ra + i) % f.head_dim % half], cs, sn);
-                    rotate_pair(va, vb, cs, sn);
-                    ya[i] = va;
-                    yb[i] = vb;
-                }
+            for (int c = 0; c < CT; ++c) acc[a][c] += sum[a][c];
+    }
+    // The K parts' sums meet in LDS (idle after the last barrier), part 0 +
+    // part 1 + ...; the KS wavefronts of a (wf, wt) share its (group, column
+    // tile) units.
+    f32x4_t* red = reinterpret_cast<f32x4_t*>(xs);   // [wavefront][tile][column][lane]
+    if constexpr (KS > 1) {
+#pragma unroll
+        for (int a = 0; a < 2 * FG; ++a)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) red[((w * 2 * FG + a) * CT + c) * 64 + lane] = acc[a][c];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int unit = 0; unit < FG * CT; ++unit) {
+        const int g_in = unit / CT, c = unit % CT;
+        if (unit % KS != part) continue;
+        f32x4_t fin[2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            if constexpr (KS > 1) {
+                const int at = ((2 * g_in + a) * CT + c) * 64 + lane;
+                constexpr int WSTEP = 2 * FG * CT * 64;
+                fin[a] = red[(wf * WT + wt) * WSTEP + at];
+#pragma unroll
+                for (int q = 1; q < KS; ++q) fin[a] += red[(q * WF * WT + wf * WT + wt) * WSTEP + at];
+            } else {
+                fin[a] = acc[2 * g_in + a][c];
             }
-            float* y = f.y[grp.m] + static_cast<int64_t>(tok) * f.n[grp.m];
-            *reinterpret_cast<f32x4_t*>(y + ra) = ya;
-            *reinterpret_cast<f32x4_t*>(y + rb) = yb;
-        } else if constexpr (MODE == FUSED_GATE_UP) {
-            const f32x4_t gv = acc[0][c] + bias4(0, ra), uv = acc[1][c] + bias4(1, ra);
-            const f32x4_t act = {swiglu_of(gv[0], uv[0]), swiglu_of(gv[1], uv[1]), swiglu_of(gv[2], uv[2]),
-                                 swiglu_of(gv[3], uv[3])};
-            *reinterpret_cast<f32x4_t*>(f.y[0] + static_cast<int64_t>(tok) * f.n[0] + ra) = act;
-        } else {
-            const int64_t row = static_cast<int64_t>(tok) * f.n[0];
-            const f32x4_t res_a = *reinterpret_cast<const f32x4_t*>(f.residual + row + ra);
-            const f32x4_t res_b = *reinterpret_cast<const f32x4_t*>(f.residual + row + rb);
-            *reinterpret_cast<f32x4_t*>(f.y[0] + row + ra) = (acc[0][c] + bias4(0, ra)) + res_a;
-            *reinterpret_cast<f32x4_t*>(f.y[0] + row + rb) = (acc[1][c] + bias4(0, rb)) + res_b;
         }
+        const int g = ftile * NG + wf * FG + g_in;
+        if (g < args.groups)
+            mm_finish<MODE>(f, mm_group<MODE>(f, g), fin[0], fin[1], tok0 + 16 * (wt * CT + c) + t, j);
     }
 }
 
@@ -1072,43 +1218,50 @@ bool mm_supported(const FusedGemv& f, int nmat, int esz, int64_t stride_k) {
 }
 
 // Launches proj_mm_kernel over `groups` feature groups (f.x already
-// normalised when the projection normalises).
-// K is split in two (twice the workgroups, half the stages each) when the
-// whole-K grid would give fewer than 256 workgroups and K is a multiple of 256.
-template <int MODE>
+// normalised when the projection normalises), with the smallest tile whose grid
+// the 256 CUs hold at once: small tiles read weights and inputs more often but
+// leave no CU idle, and past one workgroup per CU a larger tile costs less than
+// a second round.  Measured (us; tile features x tokens):
+//   K 2,048:  2,048 outputs, 100 tokens  32x32 12.2  64x32 12.1  128x64 19.6  (before 22)
+//            11,264 outputs, 100 tokens  64x32 39    128x64 26    128x128 34  (before 41)
+//            11,264 outputs, 200 tokens  128x64 46   128x128 34
+//   K 5,632:  2,048 outputs, 100 tokens  32x32 23.5  64x32 27.6  128x64 46.6  (before 54)
+//             2,048 outputs, 500 tokens  64x64 44    128x64 49   128x128 73
+// and with three parts, K 14,336, 4,096 outputs: 32 tokens 32x32 62, 100
+// tokens 64x32 81, 500 tokens 128x64 200 (before 17,700, one wavefront per
+// output and token).
+template <int MODE, int PARTS>
 int launch_mm(const FusedGemv& f, int groups, hipStream_t s) {
-    MmArgs a{f, groups, cdiv(f.rows, kMmTokens)};
-    auto grid_of = [&](int gpw) { return static_cast<int64_t>(cdiv(cdiv(groups, gpw), 8)) * 8 * a.token_tiles; };
-    auto go = [&](auto kern, int ks) {
-        const int64_t wgs = grid_of(kMmWaves / ks);
+    // A grid of feature tiles (8 at a time for the XCDs) x token tiles.
+    auto grid_of = [&](int tile_groups, int tokens) {
+        return static_cast<int64_t>(cdiv(cdiv(groups, tile_groups), 8)) * 8 * cdiv(f.rows, tokens);
+    };
+    auto go = [&](auto kern, auto shape) {
+        using Shape = decltype(shape);
+        const int64_t wgs = grid_of(Shape::kGroups, Shape::kTokens);
         SKV_REQUIRE(wgs <= INT32_MAX, "proj_mm_kernel: grid of %lld workgroups is too large",
                     static_cast<long long>(wgs));
-        const size_t lds = 2 * static_cast<size_t>(ks) * kMmPartBytes;
         const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, Shape::kLds);
         if (attr != hipSuccess) return set_error(SKV_ERR_HIP, "proj_mm_kernel: %s", hipGetErrorString(attr));
-        kern<<<static_cast<unsigned>(wgs), 64 * kMmWaves, lds, s>>>(a);
+        kern<<<static_cast<unsigned>(wgs), 64 * kMmWaves, Shape::kLds, s>>>(
+            MmArgs{f, groups, cdiv(f.rows, Shape::kTokens)});
         return check_launch("proj_mm_kernel");
     };
-    if (grid_of(kMmWaves) < 256 && f.K % 256 == 0) return go(proj_mm_kernel<MODE, 2>, 2);
-    return go(proj_mm_kernel<MODE, 1>, 1);
+#define SKV_MM(...) go(proj_mm_kernel<MODE, PARTS, __VA_ARGS__>, MmShape<PARTS, __VA_ARGS__>{})
+    constexpr int64_t kCus = 256;
+    if (grid_of(1, 32) <= kCus) return SKV_MM(1, 1, 1, 2, 8, 4);
+    if (grid_of(2, 32) <= kCus) return SKV_MM(2, 1, 1, 2, 4, 4);
+    if (grid_of(2, 64) <= kCus) return SKV_MM(1, 2, 2, 2, 4, PARTS == 3 ? 2 : 4);   // (3 parts x 4 stages spill)
+    if (grid_of(4, 64) <= kCus) return SKV_MM(2, 2, 2, 2, 2, 4);
+    return SKV_MM(2, 2, 4, 2, 1, 4);
+#undef SKV_MM
 }
 
 // ---------------------------------------------------------------------------
 // Kernels around the library GEMMs of the prompt-pass projections
 // (skv_prompt_gemm.hip): the input split before them and the epilogues after.
 // ---------------------------------------------------------------------------
-typedef __bf16 pg_bf16x2_t __attribute__((ext_vector_type(2)));
-
-// hi = bf16(v) (round to nearest even) of two values and lo = bf16 of the
-// exact remainders v - hi, packed two to a word.
-__device__ __forceinline__ void split_pair(float v0, float v1, uint32_t& hi, uint32_t& lo) {
-    const pg_bf16x2_t h = {static_cast<__bf16>(v0), static_cast<__bf16>(v1)};
-    hi = __builtin_bit_cast(uint32_t, h);
-    const pg_bf16x2_t l = {static_cast<__bf16>(v0 - bf16_lo(hi)), static_cast<__bf16>(v1 - bf16_hi(hi))};
-    lo = __builtin_bit_cast(uint32_t, l);
-}
-
 // One workgroup per row; each thread splits 4 consecutive values per pass.
 // With a RoPE table (rope.cs != nullptr) the workgroup also writes its token's
 // cos / sin per rotation pair (rope_cos_sin of position first + row), which
@@ -1305,6 +1458,24 @@ extern "C" int skv_linear_f32(const float* x, int rows, const void* weight, int 
         f.y[0] = y;
         return launch_fused<FUSED_LINEAR>(f, bf16, cdiv(out_dim, 2), s);
     }
+    // Several rows on the matrix cores (three exact bf16 parts of each input,
+    // fp32 sums).  From 5 rows: gemv_rows_vec_kernel reads the weights once per
+    // row (from L2 after the first), 15.7 / 29.0 / 42.1 us for 2 / 4 / 6 rows of
+    // 5,632 x 2,048 against 22 us for any of them here, and 6.7 / 10.4 / 13.5
+    // against 11.5 at 2,048 x 2,048.
+    if (rows >= 5 && bf16 && stride_k == 1 && in_dim % 64 == 0 && out_dim % 32 == 0 && aligned16(weight) &&
+        (stride_n * esz) % 16 == 0 && aligned16(x) && aligned16(y)) {
+        FusedGemv f{};
+        f.x = x;
+        f.rows = rows;
+        f.K = in_dim;
+        f.w[0] = weight;
+        f.row_bytes[0] = stride_n * esz;
+        f.bias[0] = bias;
+        f.n[0] = out_dim;
+        f.y[0] = y;
+        return launch_mm<FUSED_LINEAR, 3>(f, out_dim / 32, s);
+    }
     if (stride_k == 1 && aligned16(weight) && (stride_n * esz) % 16 == 0 && rows <= 64) {
         const unsigned grid = static_cast<unsigned>(cdiv(out_dim, 4 * kGemvRowsPerWave));
         const bool lds_x = static_cast<int64_t>(rows) * in_dim <= kGemvMaxLdsK;
@@ -1428,7 +1599,7 @@ int fused_qkv(const char* fn, const float* hidden, int rows, const float* gamma,
         if (position >= 0) f.rope = rope_inv_freq(head_dim);
         if (int rc = normalize_rows(fn, f.x, rows, gamma, epsilon, hidden_dim, normalized, s)) return rc;
         f.gamma = nullptr;
-        return launch_mm<FUSED_QKV>(f, (ns[0] + ns[1] + ns[2]) / 32, s);
+        return launch_mm<FUSED_QKV, 2>(f, (ns[0] + ns[1] + ns[2]) / 32, s);
     }
     if (rows == 1) {
         if (position_at != nullptr) {
@@ -1488,7 +1659,7 @@ int fused_gate_up(const char* fn, const float* x, int rows, const float* gamma, 
                              "16-byte aligned input and output", fn);
         if (int rc = normalize_rows(fn, f.x, rows, gamma, epsilon, in_dim, normalized, s)) return rc;
         f.gamma = nullptr;
-        return launch_mm<FUSED_GATE_UP>(f, out_dim / 16, s);
+        return launch_mm<FUSED_GATE_UP, 2>(f, out_dim / 16, s);
     }
     if (rows == 1) return launch_fused<FUSED_GATE_UP>(f, esz == 2, out_dim, s);
     if (!rows_supported(esz == 2, in_dim))
@@ -1527,7 +1698,7 @@ int linear_residual(const char* fn, const float* x, int rows, const void* weight
             return set_error(SKV_ERR_UNSUPPORTED,
                              "%s: needs bf16 weights, in_dim a multiple of 128, out_dim a multiple of 32 and "
                              "16-byte aligned input, residual and output", fn);
-        return launch_mm<FUSED_RESIDUAL>(f, out_dim / 32, s);
+        return launch_mm<FUSED_RESIDUAL, 2>(f, out_dim / 32, s);
     }
     if (rows == 1) return launch_fused<FUSED_RESIDUAL>(f, esz == 2, cdiv(out_dim, 2), s);
     return launch_fused_rows<FUSED_RESIDUAL>(f, esz == 2, cdiv(out_dim, 2), s);

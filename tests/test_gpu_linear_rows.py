@@ -1,0 +1,47 @@
+"""skv_linear_f32 of several rows against float64, at the edges of the matrix-core kernel's tiles (32 to 128
+tokens and outputs, stages of 32 split over 1 to 8 parts of K) and of its rule (5 rows, K a multiple of 64,
+outputs a multiple of 32, bf16 weights), and the error against the one-row kernel's."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _linear(skv, x, w_bits, bias):
+    rows, K = x.shape
+    N = w_bits.shape[0]
+    dx, dw = skv.DeviceBuffer.from_numpy(x), skv.DeviceBuffer.from_numpy(w_bits)
+    db = skv.DeviceBuffer.from_numpy(bias) if bias is not None else None
+    dy = skv.DeviceBuffer.from_numpy(np.full((rows, N), np.nan, np.float32))
+    skv._check(skv.lib().skv_linear_f32(dx.ptr, rows, dw.ptr, skv.DTYPE_BF16, 1, K, K, N, db.ptr if db else None, dy.ptr,
+                                        None))
+    skv.synchronize()
+    return dy.download(np.float32, (rows, N))
+
+
+@pytest.mark.parametrize("rows", [4, 5, 33, 64, 65, 130])
+@pytest.mark.parametrize("K,N", [(64, 32), (128, 96), (192, 64), (448, 512), (2048, 2080), (14336, 256), (64, 24576), (96, 64),
+                                 (320, 40)])
+def test_linear_rows(gpu, rows, K, N):
+    rng = np.random.default_rng(rows * 7 + K + N)
+    x = rng.standard_normal((rows, K), dtype=np.float32)
+    x[0, : K // 2] *= 1e4          # parts of very different magnitudes
+    w = oracle.f32_to_bf16(rng.standard_normal((N, K), dtype=np.float32))
+    bias = rng.standard_normal(N).astype(np.float32) if N % 64 else None
+    got = _linear(gpu, x, w, bias)
+    wf = oracle.bf16_to_f32(w).astype(np.float64)
+    ref = x.astype(np.float64) @ wf.T + (0 if bias is None else bias)
+    # fp32 sums of K products: a rounding of 2^-24 per addition, random in sign, on sums of about the
+    # products' norm; the exact split adds 3 additions per product.
+    scale = np.sqrt((x.astype(np.float64) ** 2) @ (wf ** 2).T)
+    bound = 2.0 ** -24 * (4 + 3 * np.sqrt(3 * K)) * scale + 1e-30
+    assert np.isfinite(got).all()
+    assert (np.abs(got - ref) <= bound).all(), f"worst {np.max(np.abs(got - ref) / bound):.2f} of the bound"
+    one = np.concatenate([_linear(gpu, x[r:r + 1], w, bias) for r in range(0, rows, max(1, rows // 4))])
+    pick = slice(0, rows, max(1, rows // 4))
+    err = np.linalg.norm((got[pick] - ref[pick]) / scale[pick])
+    err1 = np.linalg.norm((one - ref[pick]) / scale[pick])
+    # No less precise than the one-row kernel, up to the rounding of the result itself (2^-24 an output).
+    assert err <= 1.1 * err1 + 2.0 ** -24 * np.sqrt(one.size), f"error {err:.2e}, one row at a time {err1:.2e}"
