@@ -60,6 +60,13 @@
 //   in bf16, or infinite) has its rows recomputed in fp32 instead.
 // * Online softmax in the exp2 domain with lazy rescaling (threshold 2^8, so
 //   P <= 256 stays well inside the fp16 range).
+// * KP > 1 (grids that leave CUs idle): the workgroup owns 256 / KP rows, and
+//   KP wavefronts share each 32 of them, every one taking its 64 keys of a step
+//   of 64 KP; their outputs meet in LDS at the end.  KP times the workgroups,
+//   each with a KP-th of the steps; a step stages KP times the keys.  Chunks of
+//   273, 189 and 241 tokens over 5,725, 4,126 and 4,421 cached ones, 32 Q / 4 KV
+//   heads of 64, fp32 queries: 92 workgroups of up to 94 steps took 158 us, with
+//   KP 2 180 of up to 47 take 99.
 // Other shapes run a simple kernel (one wavefront per token and query head).
 #include "skv_common.h"
 
@@ -146,17 +153,17 @@ __device__ __forceinline__ int find_tile_seq(const int* T, int B, int tile) {
 // keys; O^T output: dims 16 dt + 4j + i, query row t.
 // ---------------------------------------------------------------------------
 constexpr int kPrefillWaves = 8;
-constexpr int kPrefillRows = kPrefillWaves * 32;   // query rows per workgroup
-constexpr int kPrefillKeys = 64;                   // keys per step
+constexpr int kPrefillRows = kPrefillWaves * 32;   // query rows per workgroup (KP = 1)
+constexpr int kPrefillKeys = 64;                   // keys per step and wavefront
 
-template <int HD>
+template <int HD, int KP>
 struct PrefillLds {
     // K rows unpadded: 16-byte chunk c of row r stored at chunk position
     // c ^ (r % chunks per row).
     static constexpr int KRS = HD * 2;             // K row stride (bytes)
     static constexpr int VRS = HD * 2 + 32;        // V row stride (bytes)
-    static constexpr int KB = kPrefillKeys * KRS;
-    static constexpr int BUF = KB + kPrefillKeys * VRS;
+    static constexpr int KB = KP * kPrefillKeys * KRS;
+    static constexpr int BUF = KB + KP * kPrefillKeys * VRS;
     static constexpr int TOTAL = 2 * BUF;          // two buffers; the tile scan follows
     __device__ static constexpr int k_chunk(int row, int c) {
         return row * KRS + (c ^ (row & (HD / 8 - 1))) * 16;
@@ -247,16 +254,17 @@ __device__ __forceinline__ void prefill_rows_fp32(const PrefillParams& p, int b,
     }
 }
 
-template <int HD, int G, bool QF32>
+template <int HD, int G, bool QF32, int KP>
 __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(PrefillParams p) {
-    using Lds = PrefillLds<HD>;
+    using Lds = PrefillLds<HD, KP>;
     constexpr int KS = kPrefillKeys;
+    constexpr int RG = kPrefillWaves / KP;   // groups of 32 rows
     static_assert(KS == 64, "one validity bit per key of a step in a 64-bit mask");
     constexpr int CH = HD / 8;              // 16-byte chunks per row
     constexpr int NKC = HD / 32;            // 32-dim steps of S
     constexpr int NDT = HD / 16;            // 16-dim tiles of O
     constexpr int QP = QF32 ? 2 : 1;
-    constexpr int QT = kPrefillRows / G;    // tokens per tile
+    constexpr int QT = 32 * RG / G;         // tokens per tile
     constexpr int NT = 64 * kPrefillWaves;
     constexpr int LOADS = KS * CH / NT;     // 16-byte chunks per thread per step (K, and V)
     static_assert(LOADS >= 1 && KS * CH % NT == 0, "load split");
@@ -268,6 +276,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int t = lane & 15, j = lane >> 4;
+    const int rg = KP == 1 ? wv : wv % RG, kp = KP == 1 ? 0 : wv / RG;   // row group, key part
     const int kvh = blockIdx.x % p.Hkv;
     const int slot = blockIdx.x / p.Hkv;
 
@@ -297,7 +306,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
     const int32_t* table = p.tables + static_cast<int64_t>(b) * p.max_blocks;
     const int64_t row_stride = static_cast<int64_t>(p.Hkv) * HD;
     // Position of this wave's first query row (its rows' positions only grow).
-    const int wave_first_pos = base_pos + (wv * 32) / G;
+    const int wave_first_pos = base_pos + (rg * 32) / G;
 
     // This lane's two query rows (column t of the two column groups).
     int qpos[2];
@@ -305,7 +314,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
     bool live[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-        const int r = wv * 32 + c * 16 + t;
+        const int r = rg * 32 + c * 16 + t;
         const int qtok = r / G, qhead = kvh * G + r % G;
         live[c] = qtok < ntok;
         qpos[c] = live[c] ? base_pos + qtok : -1;      // -1: every key masked
@@ -379,17 +388,17 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
         wmask = __ballot(ok);
     };
     set_window(tab_load(0));
-    auto window = [&](int s) {   // blocks 4 s .. 4 s + 3; steps are visited in order
-        if (4 * s - tb >= 64) {
+    auto window = [&](int s) {   // blocks 4 KP s .. 4 KP s + 4 KP - 1; steps are visited in order
+        if (4 * KP * s - tb >= 64) {
             tb += 64;
             set_window(tvn);
             tvn = tab_load(tb + 64);
         }
     };
-    // Bit hb set when block hb of step s exists.
-    auto step_nib = [&](int s) -> uint32_t { return static_cast<uint32_t>(wmask >> (4 * s - tb)) & 0xFu; };
-    // Loads of a step: wavefront wv stages rows 8 (wv & 1) .. + 7 of the
-    // step's block wv >> 1 (LOADS passes of 64 / CH rows, CH consecutive lanes
+    // Bit hb set when block hb of this wavefront's keys of step s exists.
+    auto step_nib = [&](int s) -> uint32_t { return static_cast<uint32_t>(wmask >> (4 * (KP * s + kp) - tb)) & 0xFu; };
+    // Loads of a step: wavefront wv stages rows 8 (wv & 1) .. + 7 of block
+    // wv >> 1 of each of the step's KP times 64 keys (LOADS passes of 64 / CH rows, CH consecutive lanes
     // per row slice), through a buffer descriptor that spans exactly the
     // block's existing rows (0 for an absent block), so rows that do not exist
     // load as zeros and every load is issued unconditionally.
@@ -412,24 +421,30 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
         const int lr = 16 * blk_w + row_w[u];
         kvoff_w[u] = static_cast<int>(row_w[u] * row_bytes + (((lane % CH) ^ (lr & (CH - 1))) * 16));
     }
-    auto load_step = [&](int s, int buf, u32x4_t (&vr)[LOADS]) {
-        const int slot = 4 * s + blk_w - tb;
-        const uint64_t off = static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(off_lo, slot))) |
-                             static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(off_hi, slot))) << 32;
-        const int nrec = __builtin_amdgcn_readlane(nrec_v, slot);
-        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(kbase)) + off, 0, nrec, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(vbase)) + off, 0, nrec, 0x00020000);
+    auto load_step = [&](int s, int buf, u32x4_t (&vr)[KP][LOADS]) {
         unsigned char* kb = lds + buf * Lds::BUF;
+        __amdgpu_buffer_rsrc_t rv[KP];
 #pragma unroll
-        for (int u = 0; u < LOADS; ++u) {
-            const int lr0 = 16 * blk_w + 8 * (wv & 1) + u * (64 / CH);   // first LDS row of this pass
-            lds_dma16(rk, kb + lr0 * Lds::KRS, kvoff_w[u]);
+        for (int kq = 0; kq < KP; ++kq) {
+            const int slot = 4 * (KP * s + kq) + blk_w - tb;
+            const uint64_t off = static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(off_lo, slot))) |
+                                 static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(off_hi, slot))) << 32;
+            const int nrec = __builtin_amdgcn_readlane(nrec_v, slot);
+            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(kbase)) + off, 0, nrec, 0x00020000);
+            rv[kq] = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<unsigned char*>(reinterpret_cast<const unsigned char*>(vbase)) + off, 0, nrec, 0x00020000);
+#pragma unroll
+            for (int u = 0; u < LOADS; ++u) {
+                const int lr0 = KS * kq + 16 * blk_w + 8 * (wv & 1) + u * (64 / CH);   // first LDS row of this pass
+                lds_dma16(rk, kb + lr0 * Lds::KRS, kvoff_w[u]);
+            }
         }
 #pragma unroll
-        for (int u = 0; u < LOADS; ++u)
-            vr[u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv, voff_w[u], 0, 0));
+        for (int kq = 0; kq < KP; ++kq)
+#pragma unroll
+            for (int u = 0; u < LOADS; ++u)
+                vr[kq][u] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rv[kq], voff_w[u], 0, 0));
     };
     // Rows of keys that do not exist are stored as zeros (V must not carry
     // NaN from unused slots into 0 * V).
@@ -437,16 +452,18 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
     // keep an absolute error below 2^-25); vmax tracks the largest |V| this
     // thread stored.
     float vmax = 0.0f;
-    auto store_step = [&](int buf, const u32x4_t (&vr)[LOADS]) {
+    auto store_step = [&](int buf, const u32x4_t (&vr)[KP][LOADS]) {
         unsigned char* kb = lds + buf * Lds::BUF;
         unsigned char* vb = kb + Lds::KB;
 #pragma unroll
+        for (int kq = 0; kq < KP; ++kq)
+#pragma unroll
         for (int u = 0; u < LOADS; ++u) {
-            const int lr = 16 * blk_w + row_w[u], lc = lane % CH;
+            const int lr = KS * kq + 16 * blk_w + row_w[u], lc = lane % CH;
             u32x4_t w;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float lo = __uint_as_float(vr[u][e] << 16), hi = __uint_as_float(vr[u][e] & 0xFFFF0000u);
+                const float lo = __uint_as_float(vr[kq][u][e] << 16), hi = __uint_as_float(vr[kq][u][e] & 0xFFFF0000u);
                 vmax = fmaxf(vmax, fmaxf(fabsf(lo), fabsf(hi)));
                 w[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, f16x2_t));
             }
@@ -462,8 +479,10 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
     float m[2] = {-INFINITY, -INFINITY};   // reference max of each row (log2 units)
     float lsum[2] = {0.0f, 0.0f};          // this lane's share of each row's denominator
 
-    const int nsteps = cdiv(keys_end, KS);
-    u32x4_t vr[LOADS];
+    const int nsteps = cdiv(keys_end, KP * KS);
+    // Position of this wave's last live query row: key parts past it have nothing to add.
+    const int wave_last_pos = min(base_pos + (rg * 32 + 31) / G, last_pos);
+    u32x4_t vr[KP][LOADS];
     uint32_t nib_cur = 0, nib_next = 0;   // blocks of the current and next step that exist
     if (nsteps > 0) {
         nib_cur = step_nib(0);
@@ -479,9 +498,10 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
             nib_next = step_nib(st + 1);
             load_step(st + 1, cur ^ 1, vr);
         }
-        const unsigned char* kb = lds + cur * Lds::BUF;
-        const unsigned char* vb = kb + Lds::KB;
-        const int k0 = st * KS;
+        const unsigned char* kb = lds + cur * Lds::BUF + kp * KS * Lds::KRS;
+        const unsigned char* vb = lds + cur * Lds::BUF + Lds::KB + kp * KS * Lds::VRS;
+        const int k0 = (st * KP + kp) * KS;
+        if (KP == 1 || k0 <= wave_last_pos) {
 
         // ---- S^T tiles: s[c][kt] = scores of keys 16 kt + 4j + i, row t of group c
         f32x4_t s[2][KS / 16];
@@ -581,6 +601,7 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
                     acc[dt][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pf[c][h], acc[dt][c], 0, 0, 0);
             }
         }
+        }
 
         if (st + 1 < nsteps) store_step(cur ^ 1, vr);
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);   // the next step's K rows are in LDS
@@ -593,8 +614,53 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void prefill_mfma_kernel(Prefil
     if (vmax > 65504.0f) T_s[p.B + 2] = 1;
     __syncthreads();
     if (T_s[p.B + 2] != 0) {
-        prefill_rows_fp32<HD, G, QF32>(p, b, kvh, wv, ntok, tok0, base_pos, keys_end, table);
+        if (kp == 0) prefill_rows_fp32<HD, G, QF32>(p, b, kvh, rg, ntok, tok0, base_pos, keys_end, table);
         return;
+    }
+
+    if constexpr (KP > 1) {
+        // The key parts of a row group meet in LDS (the staging buffers are
+        // idle): part 0 rescales all to the common maximum and adds them up.
+        constexpr int WORDS = 2 * (2 + 4 * NDT);   // per lane: max, sum, outputs of two rows
+        static_assert((KP - 1) * RG * WORDS * 256 <= Lds::TOTAL, "parts fit the staging buffers");
+        float* part = reinterpret_cast<float*>(lds) + ((kp > 0 ? kp - 1 : 0) * RG + rg) * WORDS * 64 + lane;
+        if (kp > 0) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                part[(c * 2) * 64] = m[c];
+                part[(c * 2 + 1) * 64] = lsum[c];
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) part[(4 + (c * NDT + dt) * 4 + i) * 64] = acc[dt][c][i];
+            }
+        }
+        __syncthreads();
+        if (kp > 0) return;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            float M = m[c];
+#pragma unroll
+            for (int q = 0; q < KP - 1; ++q) M = fmaxf(M, part[q * RG * WORDS * 64 + (c * 2) * 64]);
+            if (M == -INFINITY) continue;   // no visible key: sums and outputs are zero
+            const float own = fast_exp2(m[c] - M);
+            lsum[c] *= own;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[dt][c][i] *= own;
+#pragma unroll
+            for (int q = 0; q < KP - 1; ++q) {
+                const float* o = part + q * RG * WORDS * 64;
+                const float w = fast_exp2(o[(c * 2) * 64] - M);
+                lsum[c] = fmaf(w, o[(c * 2 + 1) * 64], lsum[c]);
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[dt][c][i] = fmaf(w, o[(4 + (c * NDT + dt) * 4 + i) * 64], acc[dt][c][i]);
+            }
+        }
     }
 
     // ---- output: O[row][dims 16 dt + 4j + i] = acc / l
@@ -698,28 +764,62 @@ __global__ __launch_bounds__(64) void prefill_generic_kernel(PrefillParams p, in
     }
 }
 
-template <int HD, int G, bool QF32>
-int launch_prefill_shape(const PrefillParams& p, unsigned grid, hipStream_t s) {
-    const size_t lds = PrefillLds<HD>::TOTAL + sizeof(int) * (static_cast<size_t>(p.B) + 3);
-    auto kern = prefill_mfma_kernel<HD, G, QF32>;
+// LDS of a launch: the staging buffers, then the tile scan.
+template <int HD, int KP>
+size_t prefill_lds(int B) {
+    return PrefillLds<HD, KP>::TOTAL + sizeof(int) * (static_cast<size_t>(B) + 3);
+}
+
+template <int HD, int G, bool QF32, int KP>
+int launch_prefill_shape(PrefillParams p, int num_tokens, hipStream_t s) {
+    p.tile_tokens = kPrefillRows / KP / G;
+    const unsigned tiles = static_cast<unsigned>(cdiv(num_tokens, p.tile_tokens) + p.B);
+    const size_t lds = prefill_lds<HD, KP>(p.B);
+    auto kern = prefill_mfma_kernel<HD, G, QF32, KP>;
     static size_t granted = 0;   // largest dynamic LDS size requested so far
     if (lds > granted) {
         SKV_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         granted = lds;
     }
-    kern<<<grid, 64 * kPrefillWaves, lds, s>>>(p);
+    kern<<<tiles * static_cast<unsigned>(p.Hkv), 64 * kPrefillWaves, lds, s>>>(p);
     return check_launch("prefill_mfma_kernel");
 }
 
+// Key parts per row: as many as keep the grid within the 256 CUs (one
+// workgroup each; a second round costs more than the shorter steps save), 2 at
+// head_dim 128 whose buffers for 4 would not fit LDS, and no more than there
+// are 64-key steps.  Where the chunks make up most of what the tables hold
+// (prompts from their start) the tiles' key counts range from few to all, and
+// two parts still gain in two rounds, heaviest tiles first.  (Chunk and context
+// lengths are on the device: the tokens and the table width stand for them.)
+// Measured (us, bf16 queries, 1 / 2 / 4 parts):
+//   32 Q / 4 KV heads of 64:   500 tokens 18.7 / 13.7 / 11.3, over 4,000 cached
+//     105 / 66 / 46; 2 x 300 over 4,000 101 / 62 / 76 (300 workgroups with 4);
+//     2,048 tokens 54 / 40 / 57; 4 x 700 tokens 25 / 32 / 52
+//   64 Q / 8 KV heads of 128:  500 over 4,000 146 / 99; 2 x 300 over 4,000
+//     141 / 171 (304 workgroups); 1,000 tokens 43 / 39; 2,048 tokens 88 / 114
+//   16 tokens, 32 Q / 4 KV heads of 64: 6.7 / 7.7 / 8.2
+template <int HD, int G, bool QF32>
+int launch_prefill_parts(const PrefillParams& p, int num_tokens, hipStream_t s) {
+    constexpr size_t kLdsPerCu = 160 * 1024;
+    constexpr int64_t kCus = 256;
+    const int64_t keys = static_cast<int64_t>(p.max_blocks) * 16;
+    const bool from_start = 2 * static_cast<int64_t>(num_tokens) >= p.B * keys;
+    auto wgs = [&](int kp) { return static_cast<int64_t>(cdiv(num_tokens, kPrefillRows / kp / G)) * p.Hkv; };
+    if constexpr (HD == 64)
+        if (wgs(4) <= kCus && keys > 128 && prefill_lds<HD, 4>(p.B) <= kLdsPerCu)
+            return launch_prefill_shape<HD, G, QF32, 4>(p, num_tokens, s);
+    if (wgs(2) <= (from_start ? 2 : 1) * kCus && keys > 64 && prefill_lds<HD, 2>(p.B) <= kLdsPerCu)
+        return launch_prefill_shape<HD, G, QF32, 2>(p, num_tokens, s);
+    return launch_prefill_shape<HD, G, QF32, 1>(p, num_tokens, s);
+}
+
 template <bool QF32>
-int launch_prefill_mfma(PrefillParams p, int num_tokens, hipStream_t s) {
+int launch_prefill_mfma(const PrefillParams& p, int num_tokens, hipStream_t s) {
     const int G = p.Hq / p.Hkv;
-    p.tile_tokens = kPrefillRows / G;
-    const unsigned tiles = static_cast<unsigned>(cdiv(num_tokens, p.tile_tokens) + p.B);
-    const unsigned grid = tiles * static_cast<unsigned>(p.Hkv);
 #define SKV_PF(HD_, G_) \
-    if (p.HD == HD_ && G == G_) return launch_prefill_shape<HD_, G_, QF32>(p, grid, s);
+    if (p.HD == HD_ && G == G_) return launch_prefill_parts<HD_, G_, QF32>(p, num_tokens, s);
     SKV_PF(64, 1) SKV_PF(64, 2) SKV_PF(64, 4) SKV_PF(64, 8) SKV_PF(64, 16)
     SKV_PF(128, 1) SKV_PF(128, 2) SKV_PF(128, 4) SKV_PF(128, 8) SKV_PF(128, 16)
 #undef SKV_PF

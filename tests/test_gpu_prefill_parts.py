@@ -1,0 +1,45 @@
+"""Prefill attention with its rows' keys split over 4, 2 or 1 wavefronts (the count follows from the call's tokens and
+kv heads), ragged chunks around the tile and step edges, against float64; blocks missing from the tables among them."""
+import numpy as np
+import pytest
+
+import oracle
+import test_gpu_prefill as base
+
+pytestmark = pytest.mark.gpu
+
+# (geometry, tokens): grids of whole 256-row tiles from a few workgroups to over 160.
+CASES = [((32, 4, 64), 70), ((64, 32, 64), 300), ((32, 32, 64), 700), ((32, 32, 64), 1200), ((32, 32, 64), 1500),
+         ((32, 4, 128), 90), ((64, 32, 128), 600), ((32, 32, 128), 1300), ((32, 32, 128), 1500), ((16, 1, 64), 33),
+         ((16, 1, 128), 17), ((8, 4, 64), 257)]
+
+
+@pytest.mark.parametrize("q_dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("geom,tokens", CASES, ids=lambda v: str(v))
+def test_prefill_key_parts(gpu, geom, tokens, q_dtype):
+    Hq, Hkv, hd = geom
+    a = tokens * 3 // 5
+    chunk = [a, 1, tokens - a - 1]
+    ctx = [a + 255, 513, tokens - a - 1]      # prior contexts that end inside steps of 64, 128 and 256 keys
+    c = base._case(Hq, Hkv, hd, 16, ctx, chunk, q_dtype, seed=tokens + hd)
+    c["tables"][0, 2] = -1                    # a block missing early, one past the pool in the longest sequence
+    c["tables"][0, 9] = c["total"] + 5
+    got = base._gpu(gpu, c)
+    G = Hq // Hkv
+    k = oracle.bf16_to_f32(c["kp"]).astype(np.float64)
+    v = oracle.bf16_to_f32(c["vp"]).astype(np.float64)
+    row = 0
+    for b, n in enumerate(chunk):
+        pos = np.arange(ctx[b])
+        ids = c["tables"][b, pos // 16]
+        ok = (ids >= 0) & (ids < c["total"])
+        kb, vb, pb = k[ids[ok], pos[ok] % 16], v[ids[ok], pos[ok] % 16], pos[ok]
+        for h in range(0, Hq, max(1, Hq // 8)):
+            q = c["q_ref"][row:row + n, h].astype(np.float64) * c["scale"]
+            s = np.where(pb[None, :] <= ctx[b] - n + np.arange(n)[:, None], q @ kb[:, h // G].T, -np.inf)
+            w = np.exp(s - s.max(1, keepdims=True))
+            ref = w @ vb[:, h // G] / w.sum(1, keepdims=True)
+            rel = np.linalg.norm(got[row:row + n, h] - ref) / np.linalg.norm(ref)
+            # Probabilities are rounded to fp16 (2^-12 each, at random), queries kept to ~17 bits.
+            assert rel <= 2.0 ** -11, f"sequence {b} head {h}: {rel:.1e}"
+        row += n
