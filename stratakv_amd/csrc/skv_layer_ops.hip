@@ -631,20 +631,19 @@ __global__ __launch_bounds__(256) void fused_gemv_kernel(FusedGemv f) {
 // normalised (rmsnorm_kernel on the host side of the call).  Each wavefront
 // keeps its two weight rows whole in registers (K = steps * STEP, steps <=
 // NU; the host checks), so the weights are read from HBM once for all
-// tokens.  Tokens go in tiles of 16: for each wave-wide step of k the
-// workgroup stages that step of the 16 inputs in LDS (two buffers, the next
+// tokens.  Tokens go in tiles of T (4, 8 or 16): for each wave-wide step of k
+// the workgroup stages that step of the T inputs in LDS (two buffers, the next
 // step loaded while this one is computed, one barrier per step) and every
-// wavefront accumulates 16 x 2 dot products.  The per-token accumulation
+// wavefront accumulates T x 2 dot products.  The per-token accumulation
 // order is PairPrefetch's and the final reduction wave_sum's, so each token's
 // outputs have the bits fused_gemv_kernel gives for that token alone; RoPE
 // rotates token m at position + m with rope_cos_sin (the host table's values).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-constexpr int kRowsTile = 16;
 
-template <bool BF16W, int MODE, int NU, int WPG>
+template <bool BF16W, int MODE, int NU, int WPG, int T>
 __global__ __launch_bounds__(64 * WPG) void fused_gemv_rows_kernel(FusedGemv f) {
     using PF = PairPrefetch<BF16W, NU, true>;  // K is a nonzero multiple of STEP
-    constexpr int STEP = PF::STEP, EPL = PF::EPL, T = kRowsTile;
+    constexpr int STEP = PF::STEP, EPL = PF::EPL;
     constexpr int Q4 = STEP / 4;                  // float4 per staged input row
     constexpr int LPT = T * Q4 / (64 * WPG);      // float4 staged per thread per step
     static_assert(LPT * 64 * WPG == T * Q4, "step staging");
@@ -660,6 +659,10 @@ __global__ __launch_bounds__(64 * WPG) void fused_gemv_rows_kernel(FusedGemv f) 
     float* const y_seg = pick3(f.y, rp.seg);
     const int n_seg = pick3(f.n, rp.seg);
     f32x4_t st[LPT];
+    // Where float4 c of a staged row lies: a lane's EPL / 4 of them 64 apart, so
+    // that each operand read takes 64 consecutive ones (16 tokens through a
+    // 2,048 / 5,632 layer 92.7 us, 93.0 with a lane's 32 bytes together).
+    auto slot = [](int c) { return c % (EPL / 4) * 64 + c / (EPL / 4); };
     auto load_step = [&](int tile, int c) __attribute__((always_inline)) {  // rows past the end repeat the last row
 #pragma unroll
         for (int i = 0; i < LPT; ++i) {
@@ -688,7 +691,10 @@ __global__ __launch_bounds__(64 * WPG) void fused_gemv_rows_kernel(FusedGemv f) 
             if (c >= steps) continue;  // (not break: the loop must unroll, pf.q[.][c] stays in registers)
             f32x4_t* buf = xs4 + (g & 1) * T * Q4;
 #pragma unroll
-            for (int i = 0; i < LPT; ++i) buf[t + i * 64 * WPG] = st[i];
+            for (int i = 0; i < LPT; ++i) {
+                const int idx = t + i * 64 * WPG, m = idx / Q4;
+                buf[m * Q4 + slot(idx - m * Q4)] = st[i];
+            }
             __syncthreads();
             // Next step (the next tile's first after the last; past the end,
             // this tile's last again: every load is issued unconditionally).
@@ -704,7 +710,7 @@ __global__ __launch_bounds__(64 * WPG) void fused_gemv_rows_kernel(FusedGemv f) 
                 float xv[EPL];
 #pragma unroll
                 for (int q = 0; q < EPL / 4; ++q) {
-                    const f32x4_t x4 = buf[m * Q4 + lane * (EPL / 4) + q];
+                    const f32x4_t x4 = buf[m * Q4 + q * 64 + lane];
                     xv[4 * q + 0] = x4[0];
                     xv[4 * q + 1] = x4[1];
                     xv[4 * q + 2] = x4[2];
@@ -717,7 +723,9 @@ __global__ __launch_bounds__(64 * WPG) void fused_gemv_rows_kernel(FusedGemv f) 
             }
             ++g;
         }
-        // Lane (r, .) = (lane >> 3, .) ends with tokens 2r and 2r + 1.
+        // Lane (r, .) = (lane >> 3, .) ends with values r N / 8 .. of N = 2 T:
+        // tokens 2r and 2r + 1 (T 16), token r (T 8), or one output of token
+        // r / 2 (T 4), which lane r ^ 1 completes.
         float v[2 * T];
 #pragma unroll
         for (int m = 0; m < T; ++m) {
@@ -725,6 +733,8 @@ __global__ __launch_bounds__(64 * WPG) void fused_gemv_rows_kernel(FusedGemv f) 
             v[2 * m + 1] = acc[m][1];
         }
         wave_sum_scatter<2 * T>(v);
+        float second = 0.0f;
+        if constexpr (T == 4) second = __shfl_xor(v[0], 8, 64);
         if (!rp.live || (lane & 7) != 0) continue;
         auto emit = [&](int m, float a, float b) __attribute__((always_inline)) {
             if (m >= rows) return;
@@ -748,8 +758,14 @@ __global__ __launch_bounds__(64 * WPG) void fused_gemv_rows_kernel(FusedGemv f) 
                 if (rp.rb != rp.ra) f.y[0][row + rp.rb] = (b + bias_of(0, rp.rb)) + f.residual[row + rp.rb];
             }
         };
-        emit(tile * T + 2 * (lane >> 3), v[0], v[1]);
-        emit(tile * T + 2 * (lane >> 3) + 1, v[2], v[3]);
+        if constexpr (T == 16) {
+            emit(tile * T + 2 * (lane >> 3), v[0], v[1]);
+            emit(tile * T + 2 * (lane >> 3) + 1, v[2], v[3]);
+        } else if constexpr (T == 8) {
+            emit(tile * T + (lane >> 3), v[0], v[1]);
+        } else {
+            if ((lane & 8) == 0) emit(tile * T + (lane >> 4), v[0], second);
+        }
     }
 }
 
@@ -805,8 +821,8 @@ template <int MODE>
 int launch_fused_rows(const FusedGemv& f, bool bf16, int items, hipStream_t s) {
     constexpr int WPG = MODE == FUSED_GATE_UP ? 8 : 4;
     const unsigned grid = static_cast<unsigned>(cdiv(items, WPG));
-    auto go = [&](auto kern, int step) {
-        const size_t lds = 2 * sizeof(float) * static_cast<size_t>(kRowsTile) * step;
+    auto go = [&](auto kern, int step, int tile) {
+        const size_t lds = 2 * sizeof(float) * static_cast<size_t>(tile) * step;
         const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                                     static_cast<int>(lds));
@@ -814,12 +830,30 @@ int launch_fused_rows(const FusedGemv& f, bool bf16, int items, hipStream_t s) {
         kern<<<grid, 64 * WPG, lds, s>>>(f);
         return check_launch("fused_gemv_rows_kernel");
     };
-    if (bf16 && f.K % 512 == 0) {
-        if (f.K <= 2048) return go(fused_gemv_rows_kernel<true, MODE, 4, WPG>, 512);
-        if (f.K <= 4096) return go(fused_gemv_rows_kernel<true, MODE, 8, WPG>, 512);
-        if (f.K <= 6144) return go(fused_gemv_rows_kernel<true, MODE, 12, WPG>, 512);
+#define SKV_ROWS(BF16_, NU_, STEP_, T_) go(fused_gemv_rows_kernel<BF16_, MODE, NU_, WPG, T_>, STEP_, T_)
+#define SKV_ROWS_BF16(NU_)                                   \
+    {                                                        \
+        if (f.rows <= 4) return SKV_ROWS(true, NU_, 512, 4); \
+        if (eights) return SKV_ROWS(true, NU_, 512, 8);      \
+        return SKV_ROWS(true, NU_, 512, 16);                 \
     }
-    if (!bf16 && f.K % 256 == 0 && f.K <= 2048) return go(fused_gemv_rows_kernel<false, MODE, 8, WPG>, 256);
+    // A tile computes all its T tokens, whether they exist or not: the T that
+    // pads least, 16 where it pads no more than 8 (a weight is widened once per
+    // tile).  A layer of 2,048 / 5,632, us with T 16 and now: 2 tokens 88.6 /
+    // 51.4, 4 89.8 / 52.8, 8 92.0 / 64.5, 17 135.8 / 111.1, 24 139.2 / 111.9.
+    // (T 4 would leave threads of fp32 weights' staging without a float4.)
+    const bool eights = f.rows <= 8 || (f.rows > 16 && f.rows <= 24);
+    if (bf16 && f.K % 512 == 0) {
+        if (f.K <= 2048) SKV_ROWS_BF16(4)
+        if (f.K <= 4096) SKV_ROWS_BF16(8)
+        if (f.K <= 6144) SKV_ROWS_BF16(12)
+    }
+    if (!bf16 && f.K % 256 == 0 && f.K <= 2048) {
+        if (eights) return SKV_ROWS(false, 8, 256, 8);
+        return SKV_ROWS(false, 8, 256, 16);
+    }
+#undef SKV_ROWS_BF16
+#undef SKV_ROWS
     return set_error(SKV_ERR_UNSUPPORTED,
                      "fused projections of several tokens need K a multiple of %d and at most %d", bf16 ? 512 : 256,
                      bf16 ? 6144 : 2048);

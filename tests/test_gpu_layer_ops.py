@@ -323,6 +323,27 @@ def test_fused_rows_match_one_token_calls(gpu, dims, dtype, with_bias):
             assert np.array_equal(got[k], want[k]), f"{k}: rows={n_rows} position={position}"
 
 
+@pytest.mark.parametrize("dims,dtype", [((1024, 16, 4, 64, 2048), "bf16"), ((1024, 16, 4, 64, 2048), "fp32"),
+                                        ((3072, 24, 8, 128, 5632), "bf16")], ids=["k1024_bf16", "k1024_fp32", "k3072"])
+@pytest.mark.parametrize("n_rows", [2, 4, 5, 8, 9, 15, 17, 20, 24, 25, 33])
+def test_fused_rows_token_tiles(gpu, dims, dtype, n_rows):
+    """Row counts around the token tiles of 4, 8 and 16: the bits of the one-token calls."""
+    H, Hq, Hkv, hd, inter = dims
+    rng = np.random.default_rng(n_rows)
+    lib, D = gpu.lib(), gpu.DeviceBuffer
+    shapes = (("q", Hq * hd, H), ("k", Hkv * hd, H), ("v", Hkv * hd, H), ("o", H, Hq * hd),
+              ("g", inter, H), ("u", inter, H), ("d", H, inter))
+    W = {n: _bf16_rows(rng, o, i) if dtype == "bf16" else (0.03 * rng.standard_normal((o, i))).astype(np.float32)
+         for n, o, i in shapes}
+    W["dtype"] = gpu.DTYPE_BF16 if dtype == "bf16" else gpu.DTYPE_FP32
+    dW = {n: D.from_numpy(W[n]) for n, _, _ in shapes}
+    x = rng.standard_normal((n_rows, H)).astype(np.float32)
+    got = _fused_calls(gpu, lib, dims, W, dW, lambda n: None, x, 11, rows_api=True)
+    want = _fused_calls(gpu, lib, dims, W, dW, lambda n: None, x, 11, rows_api=False)
+    for k in got:
+        assert np.array_equal(got[k], want[k]), k
+
+
 def test_fused_rows_refuse_unsupported_shapes(gpu):
     """in_dim not a multiple of the wave-wide step, or too long to keep the
     rows in registers: SKV_ERR_UNSUPPORTED and nothing written."""
